@@ -20,7 +20,7 @@
 //           other shapes and halo depths) and after a signed or GSF
 //           transform's last W pass, where it applies the epilogue)
 //   2D: rows A=H, E=W on (H,W); columns A=W, E=H on (W,H), the backward row
-//       and column sweeps on the 30-slice ring writing the other layout
+//       and column sweeps writing the other layout
 // B and E are the reference's in-plane axes in its neighbour order (B outer,
 // E inner), so the exact-order path visits candidates in the reference order.
 //
@@ -66,9 +66,9 @@
 namespace {
 
 constexpr float kInf = __builtin_huge_valf();
-// Deepest halo: 2D rows use up to 24 of a 64-lane window (one-wave tiles are
-// bound by the exchange, and a lone image leaves most CUs idle); 3D windows
-// of 32 rows stop at 15 by themselves.
+// Deepest halo: 2D rows use up to 30 lanes on each side of a 64-lane window (a
+// lone image leaves most CUs idle); 3D windows of 32 rows stop at 15 by
+// themselves.
 constexpr int kMaxK = 30;
 // s_sleep units (64 clocks each) between publishing a halo and first polling
 // the neighbours' publications.
@@ -76,7 +76,8 @@ constexpr int kHaloPollDelay = 20;
 // The same for 16-row windows (measured: 12 on 128 x 256 x 256 volumes, 3 %
 // faster than 24; 12 made the 32-row windows of 512^2 planes 1 % slower).
 constexpr int kHaloPollDelay16 = 12;
-// The same for one-wave row tiles (two neighbours each): 512 clocks.
+// The same for row tiles: 512 clocks (256 and 64 measured 7 and 11 % slower
+// sweeps of 512^2: more polls in the way of the publications).
 constexpr int kRowPollDelay = 8;
 // Multi-wave tiles skip the slab loads of window rows whose values at that
 // step are not exact (see load_rows).
@@ -246,28 +247,6 @@ __device__ __forceinline__ float relax(const float (&dq)[3], const float (&Iq)[3
   }
 }
 
-// New value of an element of a one-row plane: the three candidates of the
-// front row (lanes -1, 0, +1; table entries 3..5).  The six candidates of
-// rows -1 and +1, which lie outside such a plane, are skipped as the
-// reference skips out-of-range neighbours.
-template <int CT, bool LAMB1, bool FAST>
-__device__ __forceinline__ float relax_row(float dq, const float (&Iq)[CT], const float (&In)[CT], float dinit,
-                                           const float (&e1)[9], float lg) {
-  const float c3 = candidate<1, 0, CT, LAMB1>(dq, Iq, In, e1[3], lg);
-  const float c4 = candidate<1, 1, CT, LAMB1>(dq, Iq, In, e1[4], lg);
-  const float c5 = candidate<1, 2, CT, LAMB1>(dq, Iq, In, e1[5], lg);
-  if constexpr (FAST) {
-    const float m = fminf(fminf(c3, c4), c5);
-    return (m < dinit) ? m : dinit;
-  } else {
-    float nd = dinit;
-    nd = (c3 < nd) ? c3 : nd;
-    nd = (c4 < nd) ? c4 : nd;
-    nd = (c5 < nd) ? c5 : nd;
-    return nd;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Tiled persistent sweep kernel
 // ---------------------------------------------------------------------------
@@ -288,12 +267,9 @@ struct Slab {  // one prefetched slice: image rows -1..R, distance rows 0..R-1
 //   1 (XST): writes it to Dd.dxo with B contiguous (the H pass writes the
 //     (W, H, D) layout of the W pass), staging each slice's window through
 //     LDS so each store covers a run of consecutive B.
-//   2 (XSA): writes it to Dd.dxo with A contiguous: multi-wave tiles (the W
-//     pass writing the native (D, H, W) layout) stage kRunLen consecutive
-//     slices per wave in LDS so that each store covers runs of kRunLen
-//     consecutive A; one-row tiles on the deep ring (2D rows writing the
-//     column layout and back) hold each block in registers and store a run
-//     of K elements per own lane at the exchange.
+//   2 (XSA): writes it to Dd.dxo with A contiguous (the W pass writing the
+//     native (D, H, W) layout): each wave stages kRunLen consecutive slices
+//     in LDS so that each store covers runs of kRunLen consecutive A.
 // INIT: the first sweep of a transform, whose input distance is computed from
 // the mask as it is loaded (SweepDesc::init_mode).
 // COMM: kCommWaves more waves (indices NW, NW + 1, ...) that hold no rows and
@@ -310,26 +286,19 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     unsigned *__restrict__ xhist) {
   // LDS slot = ring position of the step (a compile-time index in the
   // unrolled loops, so edge addresses are immediate offsets)
-  constexpr int NWL = NW > 1 ? NW : 1;
   constexpr bool XST = XS == 1, XSA = XS == 2;
-  // A-contiguous output of multi-wave tiles (XSW, runs staged in LDS) and of
-  // one-row tiles (XSR, each block's slices held in registers)
-  constexpr bool XSR = XSA && NW == 1 && R == 1, XSW = XSA && !XSR;
-  // XSW needs the LDS for its runs: two edge slots, alternating by step
+  static_assert(NW > 1, "one-row planes run on row_sweep_kernel");
+  // XSA needs the LDS for its runs: two edge slots, alternating by step
   // parity (one barrier per step separates a slot's reads from its rewrite
   // two steps later)
-  constexpr int ES = XSW ? 2 : P;
-  __shared__ float edge_first[ES][NWL][64];
-  __shared__ float edge_last[ES][NWL][64];
-  __shared__ float edgeI_first[ES][NWL][CT][64];
-  __shared__ float edgeI_last[ES][NWL][CT][64];
+  constexpr int ES = XSA ? 2 : P;
+  __shared__ float edge_first[ES][NW][64];
+  __shared__ float edge_last[ES][NW][64];
+  __shared__ float edgeI_first[ES][NW][CT][64];
+  __shared__ float edgeI_last[ES][NW][CT][64];
   constexpr int NWR = NW * R;  // window rows
-  // one wave of one row: the plane is a single row (nB == 1), so the only
-  // neighbours are lanes -1, 0, +1 of the front row itself
-  constexpr bool ROW1 = NW == 1 && R == 1;
   static_assert(!XST || (NW > 1 && 64 % NWR == 0), "transposed output needs a multi-wave window of 16/32/64 rows");
-  static_assert(!XSW || (NW > 1 && !COMM && !INIT && NWR > 2 * P), "A-contiguous output is a plain-sweep form");
-  static_assert(!XSR || (!COMM && !INIT), "one-row deferred stores are a plain-sweep form");
+  static_assert(!XSA || (NW > 1 && !COMM && !INIT && NWR > 2 * P), "A-contiguous output is a plain-sweep form");
   __shared__ float xtile[XST ? P : 1][XST ? NWR : 1][65];
   // XSA: slot a % kRunSlots holds slice a, one 64-lane row per own row of
   // the tile (window rows K .. K + TB - 1; the host uses this form only on
@@ -337,7 +306,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // kRunPad words apart beyond their rows, so the 16 lanes that read one
   // position's run hit different banks
   constexpr int XOR = NWR - 2 * P;  // own rows at the shallowest halo (+ 1 spare row)
-  __shared__ float xrun[XSW ? kRunSlots : 1][XSW ? (XOR + 1) * 64 + kRunPad : 1];
+  __shared__ float xrun[XSA ? kRunSlots : 1][XSA ? (XOR + 1) * 64 + kRunPad : 1];
   __shared__ unsigned xhist_wg[kXHistBuckets];  // this workgroup's exchange-wait counts (measurement)
   static_assert(!COMM || (NW > 1 && NWR % kCommWaves == 0), "exchange waves serve multi-wave sweeps");
   __shared__ float xfront[COMM ? NWR : 1][64];     // COMM: the front around an exchange
@@ -396,10 +365,8 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // every K steps; it stays within the sweep only when K is a positive
   // multiple of P.  A launch that breaks this is refused before any store,
   // and so is an A-contiguous output whose own rows or staged slices would
-  // not fit its LDS ring, or (one-row tiles) whose block is not one turn of
-  // the slab ring.
-  if (K <= 0 || K % P != 0 || (ROW1 && Dd.nB != 1) ||
-      (XSW && (Dd.nTB < 2 || Dd.TB > XOR || K > kRunSlots - kRunLen + 1)) || (XSR && K != P)) {
+  // not fit its LDS ring.
+  if (K <= 0 || K % P != 0 || (XSA && (Dd.nTB < 2 || Dd.TB > XOR || K > kRunSlots - kRunLen + 1))) {
     if (threadIdx.x == 0) __hip_atomic_store(status, FG_EINVAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return;
   }
@@ -512,48 +479,26 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // prefetches and stores of steps past the end of the sweep) gets an empty
   // buffer range: its loads return 0 and its stores are dropped, without a
   // memory access.
-  // FLAT (the one-row kernels, whose steps are latency-bound): one buffer
-  // resource per array for the whole sweep, with the array as its range
-  // (nA * sA * 4 bytes), and 32-bit offsets a * sA * 4 + lane offset, so a
-  // step costs two vector adds instead of scalar resource arithmetic.  The
-  // host runs these kernels only when (nA + 32) * sA * 4 <= 2^31: then the
-  // offsets of slices just past either end (a in [-P, nA + P), P <= 32) wrap
-  // to or stay at or beyond the range, and so do the store offsets of lanes
-  // that store nothing, which are based at 2^31.
-  constexpr bool FLAT = ROW1;
   struct Cursor {
     int a;
     long long off;
-    unsigned foff;  // FLAT: off modulo 2^32
   };
   const long long dAb = (long long)dir * sA * 4;
   auto cursor_of = [&](int step) {
     const int a = a_first + step * dir;
-    const long long off = (long long)a * sA * 4;
-    return Cursor{a, off, (unsigned)off};
+    return Cursor{a, (long long)a * sA * 4};
   };
   auto advance = [&](Cursor &c) {
-    if constexpr (FLAT) {
-      c.foff += (unsigned)dAb;
-    } else {
-      c.a += dir;
-      c.off += dAb;
-    }
+    c.a += dir;
+    c.off += dAb;
   };
-  const unsigned flat_range = FLAT ? (unsigned)((long long)nA * sA * 4) : 0u;
   auto cursor_rsrc = [&](const float *base, const Cursor &c) {
-    if constexpr (FLAT) {
-      return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, flat_range, 0x00020000);
-    } else {
-      const bool in = (unsigned)c.a < (unsigned)nA;
-      return __builtin_amdgcn_make_buffer_rsrc((void *)((const char *)base + c.off), 0, in ? 0xFFFFFFF0u : 0u,
-                                               0x00020000);
-    }
+    const bool in = (unsigned)c.a < (unsigned)nA;
+    return __builtin_amdgcn_make_buffer_rsrc((void *)((const char *)base + c.off), 0, in ? 0xFFFFFFF0u : 0u,
+                                             0x00020000);
   };
-  // byte offset of a lane's element within its resource; the out-of-range
-  // offset of a lane that stores nothing
-  auto at = [&](unsigned lofs, const Cursor &c) { return FLAT ? lofs + c.foff : lofs; };
-  auto nowhere = [&](const Cursor &c) { return FLAT ? 0x80000000u + c.foff : 0xFFFFFFFFu; };
+  // the out-of-range offset of a lane that stores nothing
+  constexpr unsigned kNowhere = 0xFFFFFFFFu;
 
   // Transposed output: wave w moves window columns (w * R + k) * (64 / NWR)
   // + lane / NWR, rows lane % NWR, for k < R; the byte offset of each element
@@ -592,8 +537,8 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // value only enters candidates whose distance operand is that +inf.
   // With several waves, image rows -1 and R of a slab are the neighbour
   // waves' rows R-1 and 0: they arrive through LDS when the slab is consumed
-  // (see step), so only rows 0..R-1 are loaded.  The initial front and the
-  // one-wave kernel load all rows.
+  // (see step), so only rows 0..R-1 are loaded.  The initial front loads all
+  // rows.
   // the initialisation from the loaded mask value: fl(v*m) (mode 1) or
   // fl(v*fl(1-m)) (mode 2), by a select rather than a branch
   const bool init_inv = Dd.init_mode == 2;
@@ -616,7 +561,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // all loaded: after the exchange they are the front image of the next
   // block's first step, whose rows are all exact again.  Computed once, so
   // the steps pay nothing for it; with K > P every row is loaded.
-  constexpr int SK = (kSkipEdgeLoads && NW > 1) ? P : 1;
+  constexpr int SK = kSkipEdgeLoads ? P : 1;
   unsigned slot_ofs[SK][R];
 #pragma unroll
   for (int t = 0; t < SK; ++t)
@@ -635,10 +580,9 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
 #pragma unroll
     for (int r = 0; r < R + 2; ++r) {
       const bool slotted = SK > 1 && t >= 0 && r >= 1 && r <= R;
-      const unsigned od = slotted ? slot_ofs[t][r - 1] : at(rofs[r], cur);
-      const unsigned oi = (slotted && t < P - 1) ? slot_ofs[t][r - 1] : at(rofs[r], cur);
-      // the one-row kernel (a plane of one row) uses only its own image row
-      if (r >= r0 && r < r1 && (!ROW1 || r == 1)) {
+      const unsigned od = slotted ? slot_ofs[t][r - 1] : rofs[r];
+      const unsigned oi = (slotted && t < P - 1) ? slot_ofs[t][r - 1] : rofs[r];
+      if (r >= r0 && r < r1) {
 #pragma unroll
         for (int c = 0; c < CT; ++c)
           S.I[c][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ri[c], (int)oi, 0, 0));
@@ -648,8 +592,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     }
   };
   auto load_slab = [&](Slab<R, CT> &S, const Cursor &cur, int t) {
-    if constexpr (NW > 1) load_rows(S, cur, 1, R + 1, t);
-    else load_rows(S, cur, 0, R + 2, t);
+    load_rows(S, cur, 1, R + 1, t);
   };
 
   // per-row validity of this lane (pad positions hold +inf in the front) and
@@ -680,7 +623,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // negative window lane are replaced before use).
   int xa_a0 = -1;  // first slice of the run awaiting its stores, or -1
   auto xa_flush = [&]() {
-    if constexpr (XSW) {
+    if constexpr (XSA) {
       constexpr int LPR = kRunLen, PPI = 64 / kRunLen;
       static_assert(64 % kRunLen == 0, "run layout");
       if (xa_a0 >= 0) {
@@ -718,11 +661,11 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // moving work across it): rows the tile does not own write a spare row,
   // and the padded steps past either end (a >= -(K - 1), K <= kXsaMaxK)
   // write slots that hold no pending slice.
-  int xrow[XSW ? R : 1];
+  int xrow[XSA ? R : 1];
 #pragma unroll
-  for (int r = 0; r < (XSW ? R : 0); ++r) xrow[r] = (row_own[r] ? w * R + r - K : XOR) * 64 + lane;
+  for (int r = 0; r < (XSA ? R : 0); ++r) xrow[r] = (row_own[r] ? w * R + r - K : XOR) * 64 + lane;
   auto xa_stage = [&](const float (&v)[R], int a) {
-    if constexpr (XSW) {
+    if constexpr (XSA) {
       const int sa = (a + kRunSlots) % kRunSlots;
 #pragma unroll
       for (int r = 0; r < R; ++r) xrun[sa][xrow[r]] = v[r];
@@ -731,34 +674,6 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
       const int g = a & (kRunLen - 1);
       const bool done = (unsigned)a < (unsigned)nA && (dir < 0 ? g == 0 : g == kRunLen - 1);
       xa_a0 = done ? a - g : xa_a0;
-    }
-  };
-
-  // XSR (one-row tiles, K == P): the block's new values stay in registers
-  // (slot p = block step p) and are stored at the next exchange, after the
-  // publications, element (a, e) at Dd.dxo[e * sXe + a * sXa]: the other 2D
-  // layout (sXe = nA, sXa = 1), each own lane writing a run of K consecutive
-  // elements.  (Deferring the stores of sweeps into their own array this way
-  // measured no faster.)  Slices past either end of the
-  // sweep (the padded last block) and lanes the tile does not own get an
-  // out-of-range offset.  The host uses this form only for arrays of less
-  // than 2 GiB (nA * nE elements).
-  float xrr[XSR ? P : 1];
-  int xr_s0 = 0;  // first step of the block held in xrr
-  const unsigned xr_range = XSR ? (unsigned)((long long)nA * nE * 4) : 0u;
-  const unsigned xr_lane = XSR ? (unsigned)e * (unsigned)Dd.sXe * 4u : 0u;  // own lanes: e >= 0
-  const unsigned xr_sa4 = XSR ? (unsigned)Dd.sXa * 4u : 0u;
-  auto xr_store = [&](float v, int a) {
-    if constexpr (XSR) {
-      const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)Dd.dxo, 0, xr_range, 0x00020000);
-      const unsigned off = (lane_own && (unsigned)a < (unsigned)nA) ? xr_lane + (unsigned)a * xr_sa4 : 0xFFFFFFFFu;
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rx, (int)off, 0, 0);
-    }
-  };
-  auto xr_flush = [&]() {
-    if constexpr (XSR) {
-#pragma unroll
-      for (int p = 0; p < P; ++p) xr_store(xrr[p], a_first + (xr_s0 + p) * dir);
     }
   };
 
@@ -777,7 +692,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     const __amdgpu_buffer_rsrc_t rs = cursor_rsrc(Dd.d, c0);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const unsigned off = (row_own[r] && lane_own) ? at(rofs[r + 1], c0) : nowhere(c0);
+      const unsigned off = (row_own[r] && lane_own) ? rofs[r + 1] : kNowhere;
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(Fd[r]), rs, (int)off, 0, 0);
     }
   }
@@ -786,7 +701,6 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     for (int r = 0; r < R; ++r) xtile[P - 1][w * R + r][lane] = Fd[r];
   }
   xa_stage(Fd, a_first - dir);  // XSA: the sweep's untouched first slice
-  xr_store(Fd[0], a_first - dir);
 #pragma unroll
   for (int p = 0; p < P - 1; ++p) load_slab(S[p], cursor_of(p), p);
   // the slices that the loop stores (step s) and prefetches (step s + P - 1)
@@ -841,19 +755,16 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
         __hip_atomic_store(pub + (long long)(b - b_own0) * own_w + lane_pub, pack(Fd[r], tag), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     }
-    // XSA: a run completed in this block (one-row tiles: the block) is
-    // stored after the publications (which then leave first) and drains
+    // XSA: a run completed in this block is stored after the publications (which then leave first) and drains
     // while the wave waits to poll; the halo wait below also waits for it,
     // so every path leaves the exchange with the same loads in flight
     xa_flush();
-    xr_flush();
     // Neighbours publish at about the same moment; polling right away mostly
     // finds their values not yet visible and costs a second round trip.
     // Waiting ~1300 clocks first was measured fastest for 32-row tiles
-    // (16..28 x 64 clocks: 20 best by ~0.2 %, 28 0.5 % slower), ~770 for
-    // 16-row tiles and 512 for one-wave row tiles.
-    if constexpr (NW == 1) __builtin_amdgcn_s_sleep(kRowPollDelay);
-    else if constexpr (NWR <= 16) __builtin_amdgcn_s_sleep(kHaloPollDelay16);
+    // (16..28 x 64 clocks: 20 best by ~0.2 %, 28 0.5 % slower) and ~770 for
+    // 16-row tiles.
+    if constexpr (NWR <= 16) __builtin_amdgcn_s_sleep(kHaloPollDelay16);
     else __builtin_amdgcn_s_sleep(kHaloPollDelay);
     // Only lanes that need a halo value load (measured faster than letting
     // every lane load some in-bounds line and selecting afterwards).
@@ -917,8 +828,8 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     // (branch-free: the edge waves read their own slot and select +inf for
     // the distance; their outer image rows then only meet +inf candidates)
     float top = kInf, bot = kInf;
-    if constexpr (NW > 1) {
-      const int es = XSW ? (s & 1) : slot;
+    {
+      const int es = XSA ? (s & 1) : slot;
       edge_first[es][w][lane] = Fd[0];
       edge_last[es][w][lane] = Fd[R - 1];
 #pragma unroll
@@ -940,18 +851,8 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
       xflush((slot + P - 1) % P, s - 1);
     }
     float nd[R];
-    if constexpr (ROW1) {
-      float Iq[CT], In[CT];
 #pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        Iq[c] = Fr.I[c][1];
-        In[c] = Sl.I[c][1];
-      }
-      const float v = relax_row<CT, LAMB1, FAST>(Fd[0], Iq, In, init_of(Sl.d[0]), e1, lg);
-      nd[0] = pvalid[0] ? v : kInf;
-    }
-#pragma unroll
-    for (int r = 0; r < (ROW1 ? 0 : R); ++r) {
+    for (int r = 0; r < R; ++r) {
       float dq[3];
       dq[0] = (r == 0) ? top : Fd[r - 1];
       dq[1] = Fd[r];
@@ -972,16 +873,14 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     if constexpr (XST) {
 #pragma unroll
       for (int r = 0; r < R; ++r) xtile[slot][w * R + r][lane] = nd[r];
-    } else if constexpr (XSW) {
+    } else if constexpr (XSA) {
       xa_stage(nd, cur_st.a);
-    } else if constexpr (XSR) {
-      xrr[slot] = nd[0];  // K == P: slot is the step's index in its block
     } else {
       // a padded step's slice is outside the array: all its stores are dropped
       const __amdgpu_buffer_rsrc_t rs = cursor_rsrc(Dd.d, cur_st);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const unsigned off = (row_own[r] && lane_own) ? at(rofs[r + 1], cur_st) : nowhere(cur_st);
+        const unsigned off = (row_own[r] && lane_own) ? rofs[r + 1] : kNowhere;
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(nd[r]), rs, (int)off, 0, 0);
       }
     }
@@ -1006,7 +905,6 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   const int nblocks = (nsteps + K - 1) / K;
   for (int blk = 0;; ++blk) {
     const int s0 = blk * K;
-    xr_s0 = s0;
     for (int g = 0; g < groups - 1; ++g) {
 #pragma unroll
       for (int p = 0; p < P; ++p) step(S[p], S[(p + P - 1) % P], s0 + g * P + p, p, true);
@@ -1024,13 +922,375 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     __syncthreads();
     xflush(P - 1, nblocks * K - 1);  // the last step sits in slot P - 1
   }
-  if constexpr (XSR) xr_flush();  // the last block
-  if constexpr (XSW) {
+  if constexpr (XSA) {
     xa_flush();  // a run completed in the last block
     if (dir > 0 && ((nA - 1) & (kRunLen - 1)) != kRunLen - 1) {  // a forward sweep's partial last run
       xa_a0 = (nA - 1) & ~(kRunLen - 1);
       xa_flush();
     }
+  }
+  if (xhist) {
+    __syncthreads();
+    if (threadIdx.x < kXHistBuckets && xhist_wg[threadIdx.x]) atomicAdd(xhist + threadIdx.x, xhist_wg[threadIdx.x]);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// One-row sweeps (2D rows and columns, planes of one row)
+// ---------------------------------------------------------------------------
+
+// Waves of a row workgroup that read global memory and prepare the steps.
+constexpr int kRowProducers = 6;
+constexpr int kRowThreads = (1 + kRowProducers) * 64;
+// Halo depths with compiled kernels are the multiples of this.
+constexpr int kRowHaloStep = 6;
+// Steps that the front wave reads from LDS ahead of their use.
+constexpr int kRowAhead = 6;
+// Row workgroups per compute unit that a plan counts on at halo depth K.  LDS
+// would hold two at K = 30, but they ran slower than one at K = 24 (a 1536^2
+// image with 3 channels: 384 workgroups at K = 30 1108 us, 96 at K = 24
+// 793 us; four times 1292 lanes, 324 workgroups at K = 24 1326 us, 188 at
+// K = 18 1543 us).
+constexpr int row_groups_per_cu(int K) { return K >= 30 ? 1 : K >= 24 ? 2 : K >= 18 ? 3 : 4; }
+
+// Everything of a row tile that both kinds of wave use.
+struct RowTile {
+  int lane, e, ew0, e_own0, e_own1;
+  bool lane_valid, lane_own;
+  int nA, dir, a_first, nsteps, nblocks;
+  unsigned stride4;     // bytes of a slice (a row of lanes)
+  unsigned dstride4;    // from one step's slice to the next (modulo 2^32)
+  unsigned range;       // bytes of the array
+  unsigned lofs;        // this lane's byte offset in a slice, clamped into it
+};
+
+// Byte offset of slice a of the sweep's arrays.  Slices before the first or
+// past the last one give offsets at or beyond the array's range (the host
+// runs these kernels only when (nA + 32) * stride4 <= 2^31), so their loads
+// return 0.
+__device__ __forceinline__ unsigned row_ofs(const RowTile &T, int a) { return (unsigned)a * T.stride4 + T.lofs; }
+
+// LDS of a row workgroup: two blocks of prepared steps and of new values.
+template <int K>
+struct RowShared {
+  float4 pay[2][K][64];
+  float res[2][K][64];  // (what the front wave reads ahead past pay lies in here)
+  float spare[(K < 2 * kRowAhead ? 2 * kRowAhead - K : 0) * 128 + 1];
+  unsigned xhist[kXHistBuckets];
+};
+static_assert(sizeof(RowShared<24>) * row_groups_per_cu(24) <= 160 << 10 &&
+                  sizeof(RowShared<18>) * row_groups_per_cu(18) <= 160 << 10 &&
+                  sizeof(RowShared<12>) * row_groups_per_cu(12) <= 160 << 10,
+              "row workgroups share a CU's LDS");
+
+// The part of block b that producer pw prepares: steps pw * SP .. pw * SP + SP - 1.
+template <int SP, int CT>
+struct RowSteps {
+  float I[SP + 1][CT];  // image: the slice before the first step, then each step's
+  float d[SP];          // old distance (or the mask, initialising sweeps)
+};
+
+template <int K, int CT, bool LAMB1>
+__device__ __forceinline__ void row_produce(const SweepDesc &Dd, const RowTile &T, int pw,
+                                            float4 (*__restrict__ pay)[K][64], float (*__restrict__ res)[K][64]) {
+  constexpr int SP = K / kRowProducers;
+  const bool init = Dd.init_mode != 0, init_inv = Dd.init_mode == 2;
+  RowSteps<SP, CT> S;
+  auto load = [&](int b) {
+    const __amdgpu_buffer_rsrc_t rd =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(init ? Dd.init_src : Dd.d), 0, T.range, 0x00020000);
+    unsigned o = row_ofs(T, T.a_first + (b * K + pw * SP - 1) * T.dir);  // the slice before the first step's
+#pragma unroll
+    for (int i = 0; i <= SP; ++i, o += T.dstride4) {
+#pragma unroll
+      for (int c = 0; c < CT; ++c) {
+        const __amdgpu_buffer_rsrc_t ri =
+            __builtin_amdgcn_make_buffer_rsrc((void *)(Dd.img + c * Dd.cs), 0, T.range, 0x00020000);
+        S.I[i][c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ri, (int)o, 0, 0));
+      }
+      if (i > 0) S.d[i - 1] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rd, (int)o, 0, 0));
+    }
+  };
+  // the weighted image differences of each step's three candidates and its
+  // old distance.  Pad lanes get +inf, so their new value is +inf.  Where the
+  // old distance is NaN the differences are too, so that the front wave's
+  // plain minimum keeps it (see row_relax).
+  auto make = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < SP; ++i) {
+      float l[3];
+      l[0] = absdiff_sum<1, 0, 1, CT>(fabsf(shiftE<0, 17>(S.I[i][0]) - S.I[i + 1][0]), S.I[i], S.I[i + 1]);
+      l[1] = absdiff_sum<1, 1, 1, CT>(fabsf(S.I[i][0] - S.I[i + 1][0]), S.I[i], S.I[i + 1]);
+      l[2] = absdiff_sum<1, 2, 1, CT>(fabsf(shiftE<2, 19>(S.I[i][0]) - S.I[i + 1][0]), S.I[i], S.I[i + 1]);
+      float d = S.d[i];
+      if (init) {
+        const float t = 1.0f - d;
+        d = Dd.init_v * (init_inv ? t : d);
+      }
+      d = T.lane_valid ? d : kInf;
+      const bool keep = !T.lane_valid || __builtin_isnan(d);
+      float4 q;
+      q.x = keep ? d : (LAMB1 ? l[0] : Dd.lg * l[0]);
+      q.y = keep ? d : (LAMB1 ? l[1] : Dd.lg * l[1]);
+      q.z = keep ? d : (LAMB1 ? l[2] : Dd.lg * l[2]);
+      q.w = d;
+      pay[b & 1][pw * SP + i][T.lane] = q;
+    }
+  };
+  // block b's new values of the tile's own lanes
+  auto store = [&](int b) {
+    if (Dd.dxo) {  // the other 2D layout: runs of consecutive slices per lane
+      const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)Dd.dxo, 0, T.range, 0x00020000);
+      const int n = (T.e_own1 - T.e_own0) * K;
+      for (int k = pw * 64 + T.lane; k < n; k += kRowProducers * 64) {
+        const int el = k / K, sl = k - el * K;
+        const int s = b * K + sl;
+        const float v = res[b & 1][sl][T.e_own0 - T.ew0 + el];
+        const unsigned o = (unsigned)(T.e_own0 + el) * (unsigned)Dd.sXe * 4u +
+                           (unsigned)(T.a_first + s * T.dir) * (unsigned)Dd.sXa * 4u;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rx, (int)(s < T.nsteps ? o : 0xFFFFFFFFu), 0, 0);
+      }
+    } else {
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dd.d, 0, T.range, 0x00020000);
+      const int s0 = b * K + pw * SP;
+      unsigned o = row_ofs(T, T.a_first + s0 * T.dir);
+#pragma unroll
+      for (int i = 0; i < SP; ++i, o += T.dstride4) {
+        const float v = res[b & 1][pw * SP + i][T.lane];
+        const bool own = T.lane_own && s0 + i < T.nsteps;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rs, (int)(own ? o : 0xFFFFFFFFu), 0, 0);
+      }
+    }
+  };
+  // While the front wave runs block b: prepare b + 1, read b + 2, store
+  // b - 1.  One copy of the code serves the first and last blocks too: a
+  // launch starts with cold instruction caches, and straight-line code of
+  // its own for them cost several microseconds a sweep.
+  for (int b = -2; b <= T.nblocks; ++b) {
+    if (b >= -1 && b + 1 < T.nblocks) make(b + 1);
+    if (b + 2 < T.nblocks) load(b + 2);
+    if (b > 0) store(b - 1);
+    if (b >= -1 && b < T.nblocks) __syncthreads();
+  }
+}
+
+// One step of the front wave: the new values from the front F and the prepared
+// differences q.x, q.y, q.z (neighbours -1, 0, +1) and old distances q.w.
+// Every instruction here is on the sweep's serial chain.  FAST: v_min3 drops
+// NaN candidates, and v_min_f32 of (m, old) returns old when m is NaN; where
+// old is NaN all candidates are (the producers see to it), so the result is
+// the reference's fold without its compare and select, whose mask write and
+// read cost the chain ~13 clocks more.  Written as one block because the
+// compiler would quiet the loaded operand of a minimum with one more
+// instruction.  A lane-shifted operand must not be read within two wait
+// states of its write: the add before it (and s_nop, or a second add)
+// stands between.
+template <bool LAMB1, bool FAST>
+__device__ __forceinline__ float row_relax(float F, const float4 &q, float e1s, float e1c) {
+  if constexpr (FAST) {
+    float c3, c4, c5;
+    if constexpr (LAMB1) {
+      asm("v_add_f32 %[c4], %[F], %[q4]\n\t"
+          "s_nop 0\n\t"
+          "v_add_f32_dpp %[c3], %[F], %[q3] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+          "v_add_f32_dpp %[c5], %[F], %[q5] wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+          "v_min3_f32 %[c3], %[c3], %[c4], %[c5]\n\t"
+          "v_min_f32 %[F], %[c3], %[d]"
+          : [F] "+v"(F), [c3] "=&v"(c3), [c4] "=&v"(c4), [c5] "=&v"(c5)
+          : [q3] "v"(q.x), [q4] "v"(q.y), [q5] "v"(q.z), [d] "v"(q.w));
+    } else {
+      float ts;
+      asm("v_add_f32 %[ts], %[F], %[es]\n\t"
+          "v_add_f32 %[c4], %[F], %[ec]\n\t"
+          "v_add_f32 %[c4], %[c4], %[q4]\n\t"
+          "v_add_f32_dpp %[c3], %[ts], %[q3] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+          "v_add_f32_dpp %[c5], %[ts], %[q5] wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+          "v_min3_f32 %[c3], %[c3], %[c4], %[c5]\n\t"
+          "v_min_f32 %[F], %[c3], %[d]"
+          : [F] "+v"(F), [ts] "=&v"(ts), [c3] "=&v"(c3), [c4] "=&v"(c4), [c5] "=&v"(c5)
+          : [q3] "v"(q.x), [q4] "v"(q.y), [q5] "v"(q.z), [d] "v"(q.w), [es] "v"(e1s), [ec] "v"(e1c));
+    }
+    return F;
+  } else {
+    // candidates may be -0: folded one by one in the reference's order
+    const float ts = F + e1s;
+    const float c[3] = {shiftE<0, 81>(ts) + q.x, (F + e1c) + q.y, shiftE<2, 83>(ts) + q.z};
+    float nd = q.w;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) nd = (c[k] < nd) ? c[k] : nd;
+    return nd;
+  }
+}
+
+// A row sweep is a chain of nA - 1 dependent steps, so a tile's time is its
+// longest wave's instructions per step plus an exchange every K steps.  The
+// work that does not depend on the front (loads, image differences and
+// weights of every channel, the initialisation, pad lanes, stores) is taken
+// off the chain: wave 0, the front wave, only reads a prepared step from LDS
+// (16 bytes a lane), adds, takes the minimum and leaves the new value in LDS,
+// while the producer waves of the workgroup prepare block b + 1, read global
+// memory for block b + 2 and store block b - 1.  One barrier per block of K steps.  Window, halo and publications
+// are those of the tiled kernel with one row.
+// Measured, 512^2, one channel, K = 30: 1690 clocks of steps (56 each), ~180 to
+// publish and ~1100 until the neighbours' values are there, per block of 30
+// steps; a sweep 35 us against 43 us for one wave doing everything with its
+// steps in a 30-slice register ring (20 instructions a step); 1536^2 with 3
+// channels 97 against 225 us.  Producers in six waves: with three a 3-channel
+// block waited ~750 clocks for them.
+template <int K, bool LAMB1, bool FAST>
+__global__ __launch_bounds__(kRowThreads)
+    __attribute__((amdgpu_waves_per_eu((row_groups_per_cu(K) * (kRowThreads / 64) + 3) / 4))) void row_sweep_kernel(
+    const SweepDesc *__restrict__ descs, int ndesc, SweepDesc one, int Karg, unsigned tag_base,
+    unsigned long long *__restrict__ halo_base, int *__restrict__ status, int spin_limit,
+    unsigned *__restrict__ xhist) {
+  static_assert(K % kRowProducers == 0, "producers prepare equal parts of a block");
+  __shared__ RowShared<K> sh;
+  float4 (*const pay)[K][64] = sh.pay;
+  float (*const res)[K][64] = sh.res;
+  unsigned *const xhist_wg = sh.xhist;
+  // role 0 is the front wave: wave 3, whose SIMD holds no other wave of the
+  // workgroup, and another one in each next round of 256 workgroups, so that
+  // two front waves on one CU run on different SIMDs
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), front = 3 - ((blockIdx.x >> 8) & 3);
+  const int w = wave >= front ? wave - front : wave - front + 1 + kRowProducers;
+  const int tile = xcd_remap(blockIdx.x, gridDim.x);
+  if (xhist) {
+    if (threadIdx.x < kXHistBuckets) xhist_wg[threadIdx.x] = 0u;
+    __syncthreads();
+  }
+  SweepDesc Dd;
+  if (descs) {
+    int lo = 0, hi = ndesc - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (descs[mid].tile0 <= tile) lo = mid; else hi = mid - 1;
+    }
+    Dd = descs[lo];
+  } else {
+    Dd = one;
+  }
+  if (Karg != K || Dd.nB != 1 || Dd.C < 1 || Dd.C > 4) {
+    if (threadIdx.x == 0) __hip_atomic_store(status, FG_EINVAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  const int nTE = Dd.nTE, TE = Dd.TE, nE = Dd.nE;
+  const int te = tile - Dd.tile0;
+  RowTile T;
+  T.lane = threadIdx.x & 63;
+  T.e_own0 = te * TE;
+  T.e_own1 = min(nE, T.e_own0 + TE);
+  T.ew0 = (nTE > 1) ? T.e_own0 - K : -1;
+  T.e = T.ew0 + T.lane;
+  T.lane_valid = T.e >= 0 && T.e < nE;
+  T.lane_own = T.e >= T.e_own0 && T.e < T.e_own1;
+  T.nA = Dd.nA;
+  T.dir = Dd.dir;
+  T.nsteps = Dd.nA - 1;
+  T.nblocks = (T.nsteps + K - 1) / K;
+  T.a_first = Dd.dir > 0 ? 1 : Dd.nA - 2;
+  T.stride4 = (unsigned)Dd.sA * 4u;
+  T.dstride4 = (unsigned)Dd.dir * T.stride4;
+  T.range = (unsigned)((long long)Dd.nA * Dd.sA * 4);
+  T.lofs = (unsigned)min(max(T.e, 0), nE - 1) * 4u;
+  if (T.nsteps <= 0) return;
+
+  if (w > 0) {
+    switch (Dd.C) {
+      case 1: row_produce<K, 1, LAMB1>(Dd, T, w - 1, pay, res); break;
+      case 2: row_produce<K, 2, LAMB1>(Dd, T, w - 1, pay, res); break;
+      case 3: row_produce<K, 3, LAMB1>(Dd, T, w - 1, pay, res); break;
+      default: row_produce<K, 4, LAMB1>(Dd, T, w - 1, pay, res); break;
+    }
+  } else {
+    __builtin_amdgcn_s_setprio(3);  // ahead of producers on its SIMD
+    const int lane = T.lane;
+    const float e1s = Dd.e1[3], e1c = Dd.e1[4];
+    // the front: the sweep's untouched first slice, which an initialising
+    // sweep and one that writes the other layout also store
+    float F;
+    {
+      const bool init = Dd.init_mode != 0;
+      const __amdgpu_buffer_rsrc_t rd =
+          __builtin_amdgcn_make_buffer_rsrc((void *)(init ? Dd.init_src : Dd.d), 0, T.range, 0x00020000);
+      const int a = T.a_first - T.dir;
+      float x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rd, (int)row_ofs(T, a), 0, 0));
+      if (init) {
+        const float t = 1.0f - x;
+        x = Dd.init_v * (Dd.init_mode == 2 ? t : x);
+      }
+      F = T.lane_valid ? x : kInf;
+      // (a buffer store: a flat store in flight would make every wait for an
+      // LDS read below a wait for all of them)
+      const __amdgpu_buffer_rsrc_t rs =
+          __builtin_amdgcn_make_buffer_rsrc((void *)(Dd.dxo ? Dd.dxo : Dd.d), 0, T.range, 0x00020000);
+      const unsigned o = Dd.dxo ? (unsigned)T.e * (unsigned)Dd.sXe * 4u + (unsigned)a * (unsigned)Dd.sXa * 4u
+                                : row_ofs(T, a);
+      if (T.lane_own && (Dd.dxo || init)) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F), rs, (int)o, 0, 0);
+    }
+    // the halo: own lanes within K of a neighbour publish, the other lanes
+    // of the plane reload from the tile that owns them
+    gu64 *halo = (gu64 *)halo_base + Dd.halo0;
+    const bool pub = T.lane_own && ((te > 0 && T.e - T.e_own0 < K) || (te < nTE - 1 && T.e_own1 - 1 - T.e < K));
+    const bool need = T.lane_valid && !T.lane_own && max(T.e_own0 - T.e, T.e - (T.e_own1 - 1)) <= K;
+    const int ote = T.lane_valid ? T.e / TE : te;
+    gu64 *pub_at = halo + (long long)te * 2 * TE + (T.lane_own ? T.e - T.e_own0 : 0);
+    const gu64 *src_at = halo + (long long)ote * 2 * TE + (T.lane_valid ? T.e - ote * TE : 0);
+    bool tripped = false;
+    __syncthreads();
+    for (int b = 0;; ++b) {
+      // prepared steps are read kAhead steps early; the scheduling fences keep
+      // the reads there (left alone, the compiler moves each next to its use
+      // and the chain waits for LDS at every step)
+      constexpr int kAhead = kRowAhead;
+      static_assert(K % kAhead == 0, "the steps run in groups of kAhead");
+      const float4 *pq = &pay[b & 1][0][lane];
+      float *pr = &res[b & 1][0][lane];
+      float4 q[kAhead];
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) q[s] = pq[s * 64];
+#pragma unroll
+      for (int g = 0; g < K / kAhead; ++g) {
+        // (the last group reads on past its block, inside RowShared; unused)
+        pq += kAhead * 64;
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) {
+          __builtin_amdgcn_sched_barrier(0);
+          F = row_relax<LAMB1, FAST>(F, q[s], e1s, e1c);
+          q[s] = pq[s * 64];
+          pr[s * 64] = F;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        pr += kAhead * 64;
+      }
+      if (b + 1 >= T.nblocks) break;
+      const unsigned long long t_in = xhist ? wall_clock64() : 0ull;
+      const unsigned tag = tag_base + (unsigned)(b + 1);
+      const int hslot = ((b + 1) & 1) * TE;
+      if (pub) __hip_atomic_store(pub_at + hslot, pack(F, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();  // block b is in res, block b + 1 in pay
+      if (need) {
+        __builtin_amdgcn_s_sleep(kRowPollDelay);
+        unsigned long long x = __hip_atomic_load(src_at + hslot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // after an expiry this wave waits no more: the sweep then finishes
+        // (with wrong values, reported through the status word)
+        int spins = tripped ? spin_limit : 0;
+        while ((unsigned)(x >> 32) != tag) {
+          if (++spins > spin_limit) {
+            __hip_atomic_store(status, FG_EWATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            tripped = true;
+            break;
+          }
+          x = __hip_atomic_load(src_at + hslot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        F = __uint_as_float((unsigned)x);
+      }
+      if (xhist && lane == 0) {
+        const unsigned long long dt = wall_clock64() - t_in;
+        const int bucket = dt ? min(64 - __clzll(dt), kXHistBuckets - 1) : 0;
+        atomicAdd(&xhist_wg[bucket], 1u);
+      }
+    }
+    __syncthreads();
   }
   if (xhist) {
     __syncthreads();
@@ -1431,15 +1691,10 @@ struct Shape {
 };
 // Workgroup shapes with compiled kernels: index 0 serves 2D row sweeps
 // (one row); the others tile 3D planes (selected by fg_tuning.shape).
-constexpr Shape kShapes[] = {{1, 1, 6, 6, false},  {4, 8, 2, 2, false},  {8, 4, 3, 2, false},
+constexpr Shape kShapes[] = {{1, 1, kRowHaloStep, kRowHaloStep, false},  {4, 8, 2, 2, false},  {8, 4, 3, 2, false},
                              {16, 2, 3, 3, false}, {8, 4, 5, 2, false},  {16, 2, 5, 3, false},
                              {8, 4, 5, 2, true},   {8, 2, 5, 3, false}};
 constexpr int kNumShapes = 8;
-// One-row planes at K = 30 (a lone row, or rows few enough for one tile per
-// CU at that depth): the whole block in the slab ring, so the prefetches of
-// a block are never waited for at a loop head.
-constexpr Shape kRowDeep = {1, 1, 30, 30, false};
-constexpr int kRowDeepK = 30;
 constexpr int kAutoShape = 5;  // fastest on 512^2 planes: 16 x 2 with the deepest ring that keeps K = 5
 // 16-row windows (8 x 2): with the automatic shape and halo, a pass whose planes (3D,
 // 1-2 channels, general candidate: lamb != 1) all fit the compute units with
@@ -1466,8 +1721,7 @@ struct ShapeScope {
 Plan plan_fixed(int nB, int nE, int Kreq, int C, int shape = -1) {
   Plan p{};
   p.ok = false;
-  const Shape s = (nB == 1) ? (Kreq > kRowDeepK - kShapes[0].P12 ? kRowDeep : kShapes[0])
-                            : kShapes[shape >= 0 ? shape : g_shape];
+  const Shape s = nB == 1 ? kShapes[0] : kShapes[shape >= 0 ? shape : g_shape];
   p.NW = s.NW;
   p.R = s.R;
   p.comm = s.comm && C <= 2;  // exchange-wave kernels exist for 1-2 channels; 3-4 run the plain 8 x 4
@@ -1499,18 +1753,24 @@ Plan plan_fixed(int nB, int nE, int Kreq, int C, int shape = -1) {
 }
 
 // Plan of one sweep plane.  Kreq > 0: that halo depth, rounded up to a
-// multiple of the slab ring.  Kreq == 0 (automatic): the deepest halo
-// (fewest exchanges) whose tiles still fit one per compute unit, as a tile
-// shares its CU with no other and every tile waits for its neighbours at
+// multiple of the slab ring (a row whose tiles would not all be resident at
+// that depth takes the deepest at which they are).  Kreq == 0 (automatic):
+// the deepest halo (fewest exchanges) whose tiles still fit one per compute
+// unit (rows: row_groups_per_cu), as every tile waits for its neighbours at
 // each exchange; if even the shallowest halo needs more tiles, that one.
 Plan plan_plane(int nB, int nE, int Kreq, int C, int tile_budget) {
-  if (Kreq > 0) return plan_fixed(nB, nE, Kreq, C);
+  auto budget = [&](int K) { return nB == 1 ? tile_budget * row_groups_per_cu(K) : tile_budget; };
+  if (Kreq > 0) {
+    Plan p = plan_fixed(nB, nE, Kreq, C);
+    while (nB == 1 && p.nTE > 2 * tile_budget && p.K > p.P) p = plan_fixed(nB, nE, p.K - p.P, C);
+    return p;
+  }
   const Plan first = plan_fixed(nB, nE, 1, C);
   Plan best = first;
   for (int K = first.P; K <= kMaxK; K += first.P) {
     const Plan q = plan_fixed(nB, nE, K, C);
     if (!q.ok) break;
-    if ((long long)q.nTB * q.nTE > tile_budget) break;
+    if ((long long)q.nTB * q.nTE > budget(K)) continue;
     best = q;
   }
   return best;
@@ -1578,15 +1838,22 @@ const void *pick_kernel_nr(int C, bool lamb1, bool fast, bool init) {
   return nullptr;
 }
 
-// One-row kernels with deferred stores into the other 2D layout on the ring
-// P, 1-4 channels.
-template <int P>
-const void *pick_row_deferred(int C, bool lamb1, bool fast) {
-  switch (C) {
-    case 1: return pick_variant<1, 1, P, 1, 2>(lamb1, fast);
-    case 2: return pick_variant<1, 1, P, 2, 2>(lamb1, fast);
-    case 3: return pick_variant<1, 1, P, 3, 2>(lamb1, fast);
-    case 4: return pick_variant<1, 1, P, 4, 2>(lamb1, fast);
+// The one-row kernel of halo depth K (1-4 channels, every output form and
+// initialisation), or null.
+template <int K>
+const void *pick_row_variant(bool lamb1, bool fast) {
+  if (lamb1) return reinterpret_cast<const void *>(&row_sweep_kernel<K, true, true>);
+  return fast ? reinterpret_cast<const void *>(&row_sweep_kernel<K, false, true>)
+              : reinterpret_cast<const void *>(&row_sweep_kernel<K, false, false>);
+}
+
+const void *pick_row_kernel(int K, bool lamb1, bool fast) {
+  switch (K) {
+    case 6: return pick_row_variant<6>(lamb1, fast);
+    case 12: return pick_row_variant<12>(lamb1, fast);
+    case 18: return pick_row_variant<18>(lamb1, fast);
+    case 24: return pick_row_variant<24>(lamb1, fast);
+    case 30: return pick_row_variant<30>(lamb1, fast);
     default: return nullptr;
   }
 }
@@ -1595,15 +1862,13 @@ const void *pick_row_deferred(int C, bool lamb1, bool fast) {
 // xs selects the output form (0 own layout, 1 B contiguous, 2 A contiguous).
 // B-contiguous kernels exist for the two 5-slice-ring 3D shapes: 8 x 4 with
 // 1-2 channels, 16 x 2 with 1 channel (2 channels would exceed the LDS);
-// A-contiguous ones for both shapes with 1 channel, and for one-row tiles
-// (deferred stores) on the 30-slice ring with 1-4 channels.
+// A-contiguous ones for both shapes with 1 channel.
 constexpr int kXstMaxC = 2;
 constexpr int kXsaMaxC = 1;
 constexpr int kXsaMaxK = kRunSlots - kRunLen + 1;
 const void *pick_kernel(int NW, int R, int P, int C, bool lamb1, bool fast, int xs = 0, bool init = false,
                         bool comm = false) {
   if (xs && init) return nullptr;
-  if (xs == 2 && NW == 1 && R == 1) return (P == kRowDeepK && !comm) ? pick_row_deferred<kRowDeepK>(C, lamb1, fast) : nullptr;
   if (comm) return (NW == 8 && R == 4 && P == 5) ? pick_comm_kernel(C, lamb1, fast, xs, init) : nullptr;
   if (xs == 1) {
     if (NW == 8 && R == 4 && P == 5 && C == 1) return pick_variant<8, 4, 5, 1, 1>(lamb1, fast);
@@ -1618,8 +1883,6 @@ const void *pick_kernel(int NW, int R, int P, int C, bool lamb1, bool fast, int 
   }
 #define FG_S(nw, r, p, clo, chi) \
   if (NW == nw && R == r && P == p && C >= clo && C <= chi) return pick_kernel_nr<nw, r, p, clo, chi>(C, lamb1, fast, init);
-  FG_S(1, 1, 6, 1, 4)
-  FG_S(1, 1, 30, 1, 4)
   FG_S(4, 8, 2, 1, 4)
   FG_S(8, 4, 3, 1, 2)
   FG_S(8, 4, 5, 1, 2)
@@ -1904,7 +2167,26 @@ void destroy_graph(GraphEntry &e) {
 struct SweepJob {
   Xform *x;
   int pass;
-  int K;  // halo depth of this plane's plan (> 0)
+  int K;   // halo depth of this plane's plan (> 0)
+  int xs;  // output form (SweepDesc::dxo)
+};
+
+// What the sweeps of one launch share.  Row sweeps (row()) of any channel
+// count, output form and initialisation share a kernel: C, xs and in are 0.
+struct SweepGroup {
+  int NW, R, P, K, C;
+  bool l1, fa;
+  int xs;
+  bool in, cm;
+  bool row() const { return NW == 1; }
+  int threads() const { return row() ? kRowThreads : (NW + (cm ? kCommWaves : 0)) * 64; }
+  const void *kernel() const {
+    return row() ? pick_row_kernel(K, l1, fa) : pick_kernel(NW, R, P, C, l1, fa, xs, in, cm);
+  }
+  bool operator==(const SweepGroup &o) const {
+    return NW == o.NW && R == o.R && P == o.P && K == o.K && C == o.C && l1 == o.l1 && fa == o.fa && xs == o.xs &&
+           in == o.in && cm == o.cm;
+  }
 };
 
 struct Runner {
@@ -2035,18 +2317,17 @@ struct Runner {
     }
   }
 
-  int record_tiled(std::vector<SweepJob> &jobs, int dir, int NW, int R, int P, int C, bool lamb1, bool fast,
-                   int xs = 0, bool in = false, bool cm = false) {
+  int record_tiled(std::vector<SweepJob> &jobs, int dir, const SweepGroup &g) {
     std::vector<SweepDesc> descs;
     long long halo_used = 0;
-    int tiles = 0, max_blocks = 0, kk = -1;
+    int tiles = 0, max_blocks = 0;
     double alg = 0;
     for (auto &j : jobs) {
       SweepDesc s;
-      fill_desc(*j.x, j.pass, dir, s, xs);
+      fill_desc(*j.x, j.pass, dir, s, j.xs);
       alg += (double)(s.nA - 1) * s.nB * s.nE * (4.0 * s.C + 8.0);
       Plan p = plan_fixed(s.nB, s.nE, j.K, s.C);
-      if (!p.ok || p.NW != NW || p.R != R || p.P != P || p.comm != cm || p.K % P != 0 || (kk >= 0 && kk != p.K))
+      if (!p.ok || p.NW != g.NW || p.R != g.R || p.P != g.P || p.comm != g.cm || p.K % g.P != 0 || p.K != g.K)
         return fail(FG_EINVAL, "internal: sweep plan does not match the selected kernel");
       s.nTB = p.nTB; s.nTE = p.nTE; s.TB = p.TB; s.TE = p.TE;
       s.tile0 = tiles;
@@ -2054,7 +2335,6 @@ struct Runner {
       const int nt = p.nTB * p.nTE;
       tiles += nt;
       halo_used += (long long)nt * 2 * p.TB * p.TE;
-      kk = p.K;
       max_blocks = std::max(max_blocks, (s.nA - 1) / p.K + 1);
       descs.push_back(s);
     }
@@ -2066,10 +2346,10 @@ struct Runner {
     }
     Cmd c;
     c.type = Cmd::TILED;
-    c.kern = pick_kernel(NW, R, P, C, lamb1, fast, xs, in, cm);
+    c.kern = g.kernel();
     if (!c.kern) return fail(FG_EINVAL, "no tiled kernel for this shape");
     c.grid = tiles;
-    c.block = (NW + (cm ? kCommWaves : 0)) * 64;
+    c.block = g.threads();
     c.ndesc = (int)descs.size();
     if (c.ndesc == 1) {
       c.by_value = true;
@@ -2077,7 +2357,7 @@ struct Runner {
     } else {
       c.off = rec.put(descs.data(), descs.size() * sizeof(SweepDesc));
     }
-    c.K = kk;
+    c.K = g.K;
     c.tag_base = tag_base;
     c.alg_bytes = alg;
     rec.cmds.push_back(c);
@@ -2165,8 +2445,8 @@ struct Runner {
   // tiles still fit the device, and the shallowest one when none does, as a
   // deeper halo then only adds window arithmetic (a 32 x 64 window computes
   // 1.7 x its own tile at K = 5 and 3.9 x at K = 10; a 64-lane row 1.23 x at
-  // K = 6 and 16 x at K = 30).  3D tiles fill a CU each; 2D rows are one-wave
-  // tiles bound by latency, so they fit one per SIMD.
+  // K = 6 and 16 x at K = 30).  3D tiles fill a CU each; several row
+  // workgroups share one (row_groups_per_cu).
   std::vector<int> pass_halos(const std::vector<Xform *> &active, int pass) {
     std::vector<int> ks(active.size(), 0);
     std::vector<int> rows, planes;  // automatic 2D rows and 3D planes
@@ -2177,16 +2457,15 @@ struct Runner {
       ks[i] = plan_plane(nB, nE, K, active[i]->C, dev.cus).K;
       if (K == 0) (nB > 1 ? planes : rows).push_back((int)i);
     }
-    if (rows.size() > 1) share_halo(active, pass, rows, 4LL * dev.cus, ks);
-    if (planes.size() > 1) share_halo(active, pass, planes, dev.cus, ks);
+    if (rows.size() > 1) share_halo(active, pass, rows, ks);
+    if (planes.size() > 1) share_halo(active, pass, planes, ks);
     return ks;
   }
 
   // One halo depth per slab-ring length for the planes `idx` (channel
-  // classes use different rings): the deepest whose tiles total at most
-  // `budget`, else the shallowest.
-  void share_halo(const std::vector<Xform *> &active, int pass, const std::vector<int> &idx, long long budget,
-                  std::vector<int> &ks) {
+  // classes use different rings), all rows or all 3D planes: the deepest whose
+  // tiles fit the device, else the shallowest.
+  void share_halo(const std::vector<Xform *> &active, int pass, const std::vector<int> &idx, std::vector<int> &ks) {
     auto ring = [&](int i) {
       int nA, nB, nE;
       pass_plane(*active[i], pass, nA, nB, nE);
@@ -2198,18 +2477,19 @@ struct Runner {
     for (int P : rings) {
       int best = P;
       for (int k = P; k <= kMaxK; k += P) {
-        long long tiles = 0;
+        long long tiles = 0, budget = dev.cus;
         bool ok = true;
         for (int i : idx) {
           if (ring(i) != P) continue;
           int nA, nB, nE;
           pass_plane(*active[i], pass, nA, nB, nE);
+          if (nB == 1) budget = (long long)dev.cus * row_groups_per_cu(k);
           const Plan q = plan_fixed(nB, nE, k, active[i]->C);
           if (!q.ok) { ok = false; break; }
           tiles += (long long)q.nTB * q.nTE;
         }
-        if (!ok || tiles > budget) break;
-        best = k;
+        if (!ok) break;
+        if (tiles <= budget) best = k;
       }
       for (int i : idx)
         if (ring(i) == P) ks[i] = best;
@@ -2242,8 +2522,7 @@ struct Runner {
     ShapeScope shape_scope(pass_shape(active, pass));
     const std::vector<int> ks = pass_halos(active, pass);
     for (int dir : {+1, -1}) {
-      struct G { int NW, R, P, K, C; bool l1, fa; int xs; bool in, cm; std::vector<SweepJob> jobs; };
-      std::vector<G> groups;
+      std::vector<std::pair<SweepGroup, std::vector<SweepJob>>> groups;
       for (size_t i = 0; i < active.size(); ++i) {
         Xform *x = active[i];
         int nA, nB, nE;
@@ -2258,40 +2537,34 @@ struct Runner {
           continue;
         }
         const Plan p = plan_fixed(nB, nE, ks[i], x->C);
-        // Backward sweeps that write the next layout themselves: 3D tiles
-        // stage the own rows of a tile of several along B, and the slices of
-        // one block beyond a run; 2D one-row tiles defer a block's stores to
-        // the exchange, on the 30-slice ring with one ring turn per block.
-        // Otherwise the distance moves between layouts through a transpose.
-        const bool row_other = x->is2d && p.NW == 1 && p.R == 1 && p.P == kRowDeepK && p.K == p.P &&
-                               pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 2, in, p.comm);
+        // Backward sweeps that write the next layout themselves: 2D row tiles
+        // store every block from LDS in either layout; 3D tiles stage the own
+        // rows of a tile of several along B, and the slices of one block
+        // beyond a run.  Otherwise the distance moves between layouts through
+        // a transpose.
         int xs = 0;
         if (pass == 1 && dir < 0 && x->xst) {
           // (the pass may run on a shape without a B-contiguous kernel)
-          if (!x->is2d && pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 1, in, p.comm)) xs = 1;
-          else if (x->is2d && row_other) xs = 2;
+          if (x->is2d) xs = 2;
+          else if (p.NW > 1 && pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 1, in, p.comm)) xs = 1;
           else x->xst = false;
         }
         if (pass == 2 && dir < 0 && x->xsa) {
-          if (x->is2d ? row_other
-                      : (p.nTB > 1 && p.K <= kXsaMaxK &&
-                         pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 2, in, p.comm)))
+          if (x->is2d ||
+              (p.nTB > 1 && p.K <= kXsaMaxK && pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 2, in, p.comm)))
             xs = 2;
           else
             x->xsa = false;
         }
-        bool found = false;
-        for (auto &g : groups)
-          if (g.NW == p.NW && g.R == p.R && g.P == p.P && g.K == p.K && g.C == x->C && g.l1 == x->lamb1 &&
-              g.fa == x->fast && g.xs == xs && g.in == in && g.cm == p.comm) {
-            g.jobs.push_back({x, pass, p.K});
-            found = true;
-            break;
-          }
-        if (!found) groups.push_back({p.NW, p.R, p.P, p.K, x->C, x->lamb1, x->fast, xs, in, p.comm, {{x, pass, p.K}}});
+        const bool row = p.NW == 1;
+        const SweepGroup key{p.NW, p.R, p.P, p.K, row ? 0 : x->C, x->lamb1, x->fast, row ? 0 : xs, row ? false : in,
+                             p.comm};
+        auto g = std::find_if(groups.begin(), groups.end(), [&](const auto &q) { return q.first == key; });
+        if (g == groups.end()) g = groups.insert(groups.end(), {key, {}});
+        g->second.push_back({x, pass, p.K, xs});
       }
       for (auto &g : groups) {
-        int rc = record_group(g.jobs, dir, g.NW, g.R, g.P, g.C, g.l1, g.fa, g.xs, g.in, g.cm);
+        int rc = record_group(g.second, dir, g.first);
         if (rc) return rc;
       }
     }
@@ -2299,12 +2572,11 @@ struct Runner {
   }
 
   // A group is split into launches whose tiles can all be co-resident.
-  int record_group(std::vector<SweepJob> &jobs, int dir, int NW, int R, int P, int C, bool l1, bool fa,
-                   int xs = 0, bool in = false, bool cm = false) {
-    const void *kern = pick_kernel(NW, R, P, C, l1, fa, xs, in, cm);
+  int record_group(std::vector<SweepJob> &jobs, int dir, const SweepGroup &g) {
+    const void *kern = g.kernel();
     if (!kern) return fail(FG_EINVAL, "no tiled kernel for this shape");
     long long cap = 0;
-    int rc = coresident_groups(kern, (NW + (cm ? kCommWaves : 0)) * 64, dev, cap);
+    int rc = coresident_groups(kern, g.threads(), dev, cap);
     if (rc) return rc;
     if (max_groups > 0) cap = std::min<long long>(cap, max_groups);
     // A launch lasts as long as its longest sweep: pack planes of similar
@@ -2323,21 +2595,22 @@ struct Runner {
       Plan p = plan_fixed(nB, nE, j.K, j.x->C);
       const long long nt = (long long)p.nTB * p.nTE;
       if (nt > cap) {  // one plane alone cannot be co-resident: per-slice engine
-        if (in) return fail(FG_EINVAL, "internal: an initialising sweep was planned on the per-slice engine");
+        if (j.x->init_mode && j.x->it == 0 && j.pass == first_pass(*j.x) && dir > 0)
+          return fail(FG_EINVAL, "internal: an initialising sweep was planned on the per-slice engine");
         record_per_slice(*j.x, j.pass, dir);
         if (j.pass == 1) j.x->xst = false;  // its output stays in the native layout
         if (j.pass == 2) j.x->xsa = false;  // its output stays in the W pass layout
         continue;
       }
       if (tiles + nt > cap) {
-        if ((rc = record_tiled(chunk, dir, NW, R, P, C, l1, fa, xs, in, cm))) return rc;
+        if ((rc = record_tiled(chunk, dir, g))) return rc;
         chunk.clear();
         tiles = 0;
       }
       chunk.push_back(j);
       tiles += nt;
     }
-    if (!chunk.empty()) return record_tiled(chunk, dir, NW, R, P, C, l1, fa, xs, in, cm);
+    if (!chunk.empty()) return record_tiled(chunk, dir, g);
     return FG_OK;
   }
 
@@ -2415,10 +2688,11 @@ struct Runner {
     pass_plane(x, pass, nA, nB, nE);
     const Plan p = plan_fixed(nB, nE, K > 0 ? K : 1, x.C);
     if (!p.ok) return FG_OK;
-    const void *kern = pick_kernel(p.NW, p.R, p.P, x.C, x.lamb1, x.fast, false, true, p.comm);
+    const SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm};
+    const void *kern = g.kernel();
     if (!kern) return FG_OK;
     long long cap = 0;
-    const int rc = coresident_groups(kern, (p.NW + (p.comm ? kCommWaves : 0)) * 64, dev, cap);
+    const int rc = coresident_groups(kern, g.threads(), dev, cap);
     if (rc) return rc;
     if (max_groups > 0) cap = std::min<long long>(cap, max_groups);
     tiled = (long long)p.nTB * p.nTE <= cap;
@@ -2664,7 +2938,8 @@ size_t halo_entries_for(const std::vector<OpSpec> &ops, int K) {
     for (int p = 0; p < 3; ++p) {
       int nA, nB, nE;
       pass_plane(x, p, nA, nB, nE);
-      for (int k = (K > 0 ? K : 1); k <= (K > 0 ? K : kMaxK); ++k) {
+      const bool any = K <= 0 || nB == 1;  // depths the plan may take
+      for (int k = (any ? 1 : K); k <= (any ? kMaxK : K); ++k) {
         for (int sh : {g_shape, (g_tune.shape == 0 && K <= 0) ? kSmallPlaneShape : g_shape}) {
           Plan pl = plan_fixed(nB, nE, k, o.C, sh);
           if (!pl.ok) continue;

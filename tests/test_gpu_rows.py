@@ -1,0 +1,81 @@
+"""One-row sweeps (2D rows and columns) at the sizes where their tiling can go
+wrong, bit for bit against the oracle: lines around one window (62-65 lanes),
+partial last tiles, sweeps of one step and around one and two blocks of every
+halo depth, NaN and infinite old distances, 1-4 channels in one launch."""
+import numpy as np
+import pytest
+import torch
+
+import fastgeodis_amd as FG
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+DEPTHS = [6, 12, 18, 24, 30]
+
+
+def equal(got, want):
+    got, want = np.asarray(got, np.float32), np.asarray(want, np.float32)
+    return bool(np.all((got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))))
+
+
+@pytest.fixture(params=DEPTHS + [0])
+def depth(request, device):
+    old = FG.get_tuning()
+    FG.set_tuning(halo=request.param)
+    yield request.param
+    FG.set_tuning(**old)
+
+
+def make(rng, C, H, W, special=False):
+    img = rng.random((1, C, H, W), dtype=np.float32)
+    m = np.ones((1, 1, H, W), np.float32)
+    for _ in range(3):
+        m[0, 0, rng.integers(0, H), rng.integers(0, W)] = 0
+    if special:
+        for value in (np.nan, np.inf, -np.inf, np.nan):
+            m[0, 0, rng.integers(0, H), rng.integers(0, W)] = value
+        img[0, 0, rng.integers(0, H), rng.integers(0, W)] = np.nan
+        img[0, C - 1, rng.integers(0, H), rng.integers(0, W)] = np.inf
+    return img, m
+
+
+def sizes(K):
+    """(H, W): lines of one window and of partial last tiles, sweeps of K and
+    2K steps and one to either side."""
+    K = K or 30
+    cap = 64 - 2 * K
+    return [(2, 62), (K, 63), (K + 1, 64), (K + 2, 65), (2 * K + 1, 3 * cap + 1), (2 * K + 2, 61), (97, 2), (1, 70)]
+
+
+@pytest.mark.parametrize("lamb", [1.0, 0.5, 1.5])
+@pytest.mark.parametrize("special", [False, True], ids=["finite", "nan-inf"])
+def test_sizes(depth, lamb, special):
+    rng = np.random.default_rng(7 + depth)
+    for k, (H, W) in enumerate(sizes(depth)):
+        C = 1 + k % 4
+        img, m = make(rng, C, H, W, special)
+        print(f"rows K={depth} lamb={lamb} C={C} {H}x{W} special={special}", flush=True)
+        with np.errstate(all="ignore"):
+            want = oracle.py_geodesic2d(img, m, 1e10, lamb, 2)
+        got = FG.generalised_geodesic2d(torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda(), 1e10, lamb, 2)
+        assert equal(got.cpu().numpy(), want)
+
+
+def test_channels_share_a_launch(depth):
+    rng = np.random.default_rng(11)
+    insts, wants = [], []
+    for k in range(12):
+        C, H, W = 1 + k % 4, int(rng.integers(2, 200)), int(rng.integers(2, 200))
+        op = ("unsigned", "signed", "gsf")[k % 3]
+        img, m = make(rng, C, H, W)
+        if op != "unsigned":
+            m = (rng.random((1, 1, H, W)) > 0.5).astype(np.float32)
+        insts.append(FG.Instance(torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda(), 1e10, 1.0, iter=1 + k % 2,
+                                 op=op, theta=0.1))
+        want = {"unsigned": lambda: oracle.py_geodesic2d(img, m, 1e10, 1.0, 1 + k % 2),
+                "signed": lambda: oracle.py_signed_geodesic2d(img, m, 1e10, 1.0, 1 + k % 2),
+                "gsf": lambda: oracle.py_gsf2d(img, m, 0.1, 1e10, 1.0, 1 + k % 2)}[op]()
+        wants.append(want)
+    for got, want in zip(FG.geodesic_batch(insts), wants):
+        assert equal(got.cpu().numpy(), want)
