@@ -59,6 +59,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "fastgeodis_hip.h"
@@ -215,37 +216,49 @@ __device__ __forceinline__ float candidate(float dq, const float (&Iq)[CT], cons
   }
 }
 
+// The three candidates from front row I (its distance dq and image Iq).
 template <int I, int CT, bool LAMB1>
-__device__ __forceinline__ void candidates_row(float (&c)[9], float dq, const float (&Iq)[CT],
+__device__ __forceinline__ void candidates_row(float (&c)[3], float dq, const float (&Iq)[CT],
                                                const float (&In)[CT], const float (&e1)[9], float lg) {
-  c[I * 3 + 0] = candidate<I, 0, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 0], lg);
-  c[I * 3 + 1] = candidate<I, 1, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 1], lg);
-  c[I * 3 + 2] = candidate<I, 2, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 2], lg);
+  c[0] = candidate<I, 0, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 0], lg);
+  c[1] = candidate<I, 1, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 1], lg);
+  c[2] = candidate<I, 2, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 2], lg);
 }
 
-// New value of one row element.  dq[i] / Iq[i][c]: front rows at B offset
-// i-1 (unshifted); In[c] / dinit: the element's own new-slice values.
-template <int CT, bool LAMB1, bool FAST>
-__device__ __forceinline__ float relax(const float (&dq)[3], const float (&Iq)[3][CT],
-                                       const float (&In)[CT], float dinit, const float (&e1)[9],
-                                       float lg) {
-  float c[9];
-  candidates_row<0, CT, LAMB1>(c, dq[0], Iq[0], In, e1, lg);
-  candidates_row<1, CT, LAMB1>(c, dq[1], Iq[1], In, e1, lg);
-  candidates_row<2, CT, LAMB1>(c, dq[2], Iq[2], In, e1, lg);
-  if constexpr (FAST) {
-    float m = fminf(fminf(c[0], c[1]), c[2]);
-    m = fminf(fminf(m, c[3]), c[4]);
-    m = fminf(fminf(m, c[5]), c[6]);
-    m = fminf(fminf(m, c[7]), c[8]);
-    return (m < dinit) ? m : dinit;
-  } else {
+// The nine candidates of one row element in the order they become available:
+// rows[k] is the front row (B offset + 1) of the k-th triple.
+// FAST: folded with IEEE minNum as they come (any order gives the same value,
+// as no candidate is -0); otherwise kept for the reference's order.
+template <bool FAST>
+struct Fold {
+  float c[9];   // !FAST: candidate of front row i, lane offset j at i * 3 + j
+  float m;      // FAST: minimum so far
+  float left;   // FAST: a candidate that waits for the next pair
+  int n = 0;    // triples taken
+  __device__ __forceinline__ void take(int i, const float (&t)[3]) {
+    if constexpr (FAST) {
+      if (n == 0) {
+        m = fminf(fminf(t[0], t[1]), t[2]);
+      } else if (n == 1) {
+        m = fminf(fminf(m, t[0]), t[1]);
+        left = t[2];
+      } else {
+        m = fminf(fminf(m, left), t[0]);
+        m = fminf(fminf(m, t[1]), t[2]);
+      }
+      ++n;
+    } else {
+      for (int j = 0; j < 3; ++j) c[i * 3 + j] = t[j];
+    }
+  }
+  __device__ __forceinline__ float with(float dinit) const {
+    if constexpr (FAST) return (m < dinit) ? m : dinit;
     float nd = dinit;
 #pragma unroll
     for (int k = 0; k < 9; ++k) nd = (c[k] < nd) ? c[k] : nd;
     return nd;
   }
-}
+};
 
 // ---------------------------------------------------------------------------
 // Tiled persistent sweep kernel
@@ -284,14 +297,15 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     const SweepDesc *__restrict__ descs, int ndesc, SweepDesc one, int K, unsigned tag_base,
     unsigned long long *__restrict__ halo_base, int *__restrict__ status, int spin_limit,
     unsigned *__restrict__ xhist) {
-  // LDS slot = ring position of the step (a compile-time index in the
-  // unrolled loops, so edge addresses are immediate offsets)
   constexpr bool XST = XS == 1, XSA = XS == 2;
   static_assert(NW > 1, "one-row planes run on row_sweep_kernel");
-  // XSA needs the LDS for its runs: two edge slots, alternating by step
-  // parity (one barrier per step separates a slot's reads from its rewrite
-  // two steps later)
-  constexpr int ES = XSA ? 2 : P;
+  // LDS slots of the edge rows (and of a B-contiguous window): a slot's reads
+  // and its next rewrite must be at least two steps apart (one barrier per
+  // step), so ring positions alternate between two slots and the last
+  // position of an odd ring has a third.  XSA needs the LDS for its runs: two
+  // slots, alternating by step parity.
+  constexpr int ES = (XSA || P % 2 == 0) ? 2 : 3;
+  auto edge_slot = [](int position) constexpr { return (P % 2 == 1 && position == P - 1) ? 2 : position % 2; };
   __shared__ float edge_first[ES][NW][64];
   __shared__ float edge_last[ES][NW][64];
   __shared__ float edgeI_first[ES][NW][CT][64];
@@ -299,7 +313,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   constexpr int NWR = NW * R;  // window rows
   static_assert(!XST || (NW > 1 && 64 % NWR == 0), "transposed output needs a multi-wave window of 16/32/64 rows");
   static_assert(!XSA || (NW > 1 && !COMM && !INIT && NWR > 2 * P), "A-contiguous output is a plain-sweep form");
-  __shared__ float xtile[XST ? P : 1][XST ? NWR : 1][65];
+  __shared__ float xtile[XST ? ES : 1][XST ? NWR : 1][65];
   // XSA: slot a % kRunSlots holds slice a, one 64-lane row per own row of
   // the tile (window rows K .. K + TB - 1; the host uses this form only on
   // planes of several tiles along B, where TB <= NWR - 2K); the slots are
@@ -374,6 +388,13 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   if (nsteps <= 0) return;
   const int a_first = (dir > 0) ? 1 : nA - 2;
   const int nblocks_all = (nsteps + K - 1) / K;
+
+  // Last wave with rows in the plane; later ones leave now (their rows are
+  // never read: wave w_last takes its lower neighbour row as outside), unless
+  // they still move staged windows or exchange halos.
+  const int w_last = min(NW - 1, (nB - 1 - bw0) / R);
+  if constexpr (!XST && !COMM)
+    if (w > w_last) return;
 
   // The exchange wave: the same barrier sequence as the compute waves (one
   // per step, two per exchange), publishing and polling between the two
@@ -677,6 +698,19 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     }
   };
 
+  // At block step j only rows within K - j of the tile's own rows can still
+  // reach them by the next exchange, so a wave computes in its first
+  // live_steps steps of a block: K with an own row, K less its distance to
+  // them otherwise, 0 without a row in the plane.  (It still passes its edge
+  // rows on: the neighbour wave's next step needs the last ones.)  At K = 10,
+  // where a 32-row window holds 12 own rows, this is a quarter of the work.
+  int live_steps = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int b = rb[r + 1];
+    if (b >= 0 && b < nB) live_steps = max(live_steps, K - max(max(b_own0 - b, b - (b_own1 - 1)), 0));
+  }
+
   // Slab ring: the slab of step s is S[s % P]; its image rows are also the
   // front image of step s + 1, so a slab is refilled (with the slice of step
   // s + P) only after step s + 1 has used it; the front of step 0 starts in
@@ -698,13 +732,33 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   }
   if constexpr (XST) {  // stage the first slice as step -1 (ring slot P - 1)
 #pragma unroll
-    for (int r = 0; r < R; ++r) xtile[P - 1][w * R + r][lane] = Fd[r];
+    for (int r = 0; r < R; ++r) xtile[edge_slot(P - 1)][w * R + r][lane] = Fd[r];
   }
   xa_stage(Fd, a_first - dir);  // XSA: the sweep's untouched first slice
 #pragma unroll
   for (int p = 0; p < P - 1; ++p) load_slab(S[p], cursor_of(p), p);
   // the slices that the loop stores (step s) and prefetches (step s + P - 1)
   Cursor cur_st = cursor_of(0), cur_pf = cursor_of(P - 1);
+
+  // Own-layout output of the slice at cursor c, whose values the front holds:
+  // raw buffer stores; non-own lanes get an out-of-range offset and the
+  // hardware drops their writes, and so do rows the tile does not own on the
+  // short rings.  On the 5-slice ring those rows branch around the store
+  // (512^3: 611 against 631 us a sweep; on the 3-slice ring the branch makes
+  // the waits for the prefetched slabs conservative: 919 against 811 us).  A
+  // padded step's slice is outside the array: all its stores are dropped.
+  auto store_own = [&](const Cursor &c) {
+    const __amdgpu_buffer_rsrc_t rs = cursor_rsrc(Dd.d, c);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const unsigned off = (row_own[r] && lane_own) ? rofs[r + 1] : kNowhere;
+      if (P < 5 || row_own[r]) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(Fd[r]), rs, (int)off, 0, 0);
+    }
+  };
+  // the stores that the block's last step left
+  auto store_last = [&]() {
+    if constexpr (XS == 0) store_own(Cursor{cur_st.a - dir, cur_st.off - dAb});
+  };
 
   // Publishes the tile's own front values that neighbours read and reloads
   // the halo positions of the window from the neighbours' publications.
@@ -722,6 +776,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     (void)blk;
 #pragma unroll
     for (int r = 0; r < R; ++r) xfront[w * R + r][lane] = Fd[r];
+    store_last();
     load_slab(pf_slab, cur_pf, P - 2);
     advance(cur_pf);
     __syncthreads();  // front visible to the exchange wave
@@ -759,6 +814,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     // while the wave waits to poll; the halo wait below also waits for it,
     // so every path leaves the exchange with the same loads in flight
     xa_flush();
+    store_last();
     // Neighbours publish at about the same moment; polling right away mostly
     // finds their values not yet visible and costs a second round trip.
     // Waiting ~1300 clocks first was measured fastest for 32-row tiles
@@ -819,73 +875,86 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // One slice: Sl holds the new slice (ring slot `slot`), Fr the previous
   // one (front image).  Afterwards Fr is refilled with the slice of step
   // s + P - 1.
-  auto step = [&](Slab<R, CT> &Sl, Slab<R, CT> &Fr, int s, int slot, bool prefetch) {
+  // j: its number in the block (1..K); the block's last step (no prefetch)
+  // leaves its own-layout stores to the exchange, after the publications.
+  auto step = [&](Slab<R, CT> &Sl, Slab<R, CT> &Fr, int s, int j, int slot, bool prefetch) {
     // steps past the end of the sweep (the last block is padded to K steps)
     // compute on slices of zeros and store nothing
     (void)s;
-    // wave-boundary front rows through LDS, and the new slice's image rows
+    // Wave-boundary front rows through LDS, and the new slice's image rows
     // -1 and R (the front image of the next step) from the neighbour waves
     // (branch-free: the edge waves read their own slot and select +inf for
-    // the distance; their outer image rows then only meet +inf candidates)
-    float top = kInf, bot = kInf;
-    {
-      const int es = XSA ? (s & 1) : slot;
-      edge_first[es][w][lane] = Fd[0];
-      edge_last[es][w][lane] = Fd[R - 1];
+    // the distance; their outer image rows then only meet +inf candidates).
+    // The candidates whose front row the wave holds itself are computed
+    // between the writes and the barrier, so that neither the writes' latency
+    // nor the slowest wave's barrier is idle time, and the image differences
+    // to the neighbours' rows while the reads are under way.
+    const int es = XSA ? (s & 1) : edge_slot(slot);
+    edge_first[es][w][lane] = Fd[0];
+    edge_last[es][w][lane] = Fd[R - 1];
 #pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        edgeI_first[es][w][c][lane] = Sl.I[c][1];
-        edgeI_last[es][w][c][lane] = Sl.I[c][R];
-      }
-      __syncthreads();
-      const float t = edge_last[es][max(w - 1, 0)][lane];
-      const float u = edge_first[es][min(w + 1, NW - 1)][lane];
-      top = (w > 0) ? t : kInf;
-      bot = (w < NW - 1) ? u : kInf;
-#pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        Sl.I[c][0] = edgeI_last[es][max(w - 1, 0)][c][lane];
-        Sl.I[c][R + 1] = edgeI_first[es][min(w + 1, NW - 1)][c][lane];
-      }
-      // the previous step's staged window is complete (barrier above)
-      xflush((slot + P - 1) % P, s - 1);
+    for (int c = 0; c < CT; ++c) {
+      edgeI_first[es][w][c][lane] = Sl.I[c][1];
+      edgeI_last[es][w][c][lane] = Sl.I[c][R];
     }
-    float nd[R];
+    float In[R][CT];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      float dq[3];
-      dq[0] = (r == 0) ? top : Fd[r - 1];
-      dq[1] = Fd[r];
-      dq[2] = (r == R - 1) ? bot : Fd[r + 1];
-      float Iq[3][CT], In[CT];
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        Iq[0][c] = Fr.I[c][r];
-        Iq[1][c] = Fr.I[c][r + 1];
-        Iq[2][c] = Fr.I[c][r + 2];
-        In[c] = Sl.I[c][r + 1];
-      }
-      const float v = relax<CT, LAMB1, FAST>(dq, Iq, In, init_of(Sl.d[r]), e1, lg);
-      nd[r] = pvalid[r] ? v : kInf;
-    }
-    // own outputs: raw buffer stores, non-own lanes and rows get an
-    // out-of-range offset and the hardware drops their writes (no branch)
-    if constexpr (XST) {
+      for (int c = 0; c < CT; ++c) In[r][c] = Sl.I[c][r + 1];
+    auto front_image = [&](int row, float (&Iq)[CT]) {  // image row -1..R of the previous slice
 #pragma unroll
-      for (int r = 0; r < R; ++r) xtile[slot][w * R + r][lane] = nd[r];
-    } else if constexpr (XSA) {
-      xa_stage(nd, cur_st.a);
-    } else {
-      // a padded step's slice is outside the array: all its stores are dropped
-      const __amdgpu_buffer_rsrc_t rs = cursor_rsrc(Dd.d, cur_st);
+      for (int c = 0; c < CT; ++c) Iq[c] = Fr.I[c][row + 1];
+    };
+    Fold<FAST> fold[R];
+    // triples of row r from front row r + I - 1, whose distance is dq
+    auto triple = [&](auto I_, int r, float dq) {
+      constexpr int I = decltype(I_)::value;
+      float Iq[CT], t[3];
+      front_image(r + I - 1, Iq);
+      candidates_row<I, CT, LAMB1>(t, dq, Iq, In[r], e1, lg);
+      fold[r].take(I, t);
+    };
+    constexpr std::integral_constant<int, 0> above{};
+    constexpr std::integral_constant<int, 1> same{};
+    constexpr std::integral_constant<int, 2> below{};
+    const bool live = j <= live_steps;
+    if (live) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const unsigned off = (row_own[r] && lane_own) ? rofs[r + 1] : kNowhere;
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(nd[r]), rs, (int)off, 0, 0);
+        triple(same, r, Fd[r]);
+        if (r > 0) triple(above, r, Fd[r - 1]);
+        if (r < R - 1) triple(below, r, Fd[r + 1]);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);  // (the compiler would move these past the barrier)
+    __syncthreads();
+    const float t = edge_last[es][max(w - 1, 0)][lane];
+    const float u = edge_first[es][min(w + 1, NW - 1)][lane];
 #pragma unroll
-    for (int r = 0; r < R; ++r) Fd[r] = nd[r];
+    for (int c = 0; c < CT; ++c) {
+      Sl.I[c][0] = edgeI_last[es][max(w - 1, 0)][c][lane];
+      Sl.I[c][R + 1] = edgeI_first[es][min(w + 1, NW - 1)][c][lane];
+    }
+    // the previous step's staged window is complete (barrier above)
+    xflush(edge_slot((slot + P - 1) % P), s - 1);
+    if (live) {
+      triple(above, 0, (w > 0) ? t : kInf);
+      triple(below, R - 1, (w < w_last) ? u : kInf);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float v = fold[r].with(init_of(Sl.d[r]));
+        Fd[r] = pvalid[r] ? v : kInf;
+      }
+    }
+    if constexpr (XST) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) xtile[edge_slot(slot)][w * R + r][lane] = Fd[r];
+    } else if constexpr (XSA) {
+      xa_stage(Fd, cur_st.a);
+    } else if (prefetch) {
+      store_own(cur_st);
+    }
     advance(cur_st);
     // prefetch without a branch: past the end of the sweep the loads return 0
     // and the data is never consumed (only steps that store nothing use it)
@@ -907,20 +976,23 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     const int s0 = blk * K;
     for (int g = 0; g < groups - 1; ++g) {
 #pragma unroll
-      for (int p = 0; p < P; ++p) step(S[p], S[(p + P - 1) % P], s0 + g * P + p, p, true);
+      for (int p = 0; p < P; ++p) step(S[p], S[(p + P - 1) % P], s0 + g * P + p, g * P + p + 1, p, true);
     }
     const int sl = s0 + K - P;
 #pragma unroll
-    for (int p = 0; p < P - 1; ++p) step(S[p], S[(p + P - 1) % P], sl + p, p, true);
-    step(S[P - 1], S[P - 2], sl + P - 1, P - 1, false);
-    if (blk + 1 >= nblocks) break;
+    for (int p = 0; p < P - 1; ++p) step(S[p], S[(p + P - 1) % P], sl + p, K - P + p + 1, p, true);
+    step(S[P - 1], S[P - 2], sl + P - 1, K, P - 1, false);
+    if (blk + 1 >= nblocks) {
+      store_last();
+      break;
+    }
     // deferred prefetch of step s0 + K - 1: the slice of step s0 + K + P - 2
     if constexpr (COMM) exchange_via_comm(blk + 1, S[P - 2]);
     else exchange(blk + 1, S[P - 2]);
   }
   if constexpr (XST) {
     __syncthreads();
-    xflush(P - 1, nblocks * K - 1);  // the last step sits in slot P - 1
+    xflush(edge_slot(P - 1), nblocks * K - 1);  // the last step sits in slot P - 1
   }
   if constexpr (XSA) {
     xa_flush();  // a run completed in the last block
