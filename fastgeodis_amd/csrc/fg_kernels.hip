@@ -72,11 +72,17 @@ constexpr float kInf = __builtin_huge_valf();
 // themselves.
 constexpr int kMaxK = 30;
 // s_sleep units (64 clocks each) between publishing a halo and first polling
-// the neighbours' publications.
-constexpr int kHaloPollDelay = 20;
-// The same for 16-row windows (measured: 12 on 128 x 256 x 256 volumes, 3 %
-// faster than 24; 12 made the 32-row windows of 512^2 planes 1 % slower).
-constexpr int kHaloPollDelay16 = 12;
+// the neighbours' publications, and between polls.  A poll that comes too
+// early costs a second round trip behind everything the CU has in flight, and
+// polls slow the publications down.  32-row windows, 512^2 planes (K = 5, the
+// memory system busy): a sweep took 615, 584, 577 and 582 us with 20, 28, 36
+// and 44 units, and 563 us with 36 and 8 between polls.  At K = 10 (256^2
+// planes, most CUs idle) 90.7, 89.4, 89.8 and 92.1 us with 16, 20, 28 and 36.
+constexpr int kHaloPollDelay = 36, kHaloRepollDelay = 8;
+constexpr int kHaloPollDelayDeep = 24;
+// 16-row windows (256^2 planes, K = 5): 87.0, 84.1, 88.8 and 94.3 us with 16,
+// 20, 28 and 36 units, 88.9 us with 20 and 8 between polls.
+constexpr int kHaloPollDelay16 = 20, kHaloRepollDelay16 = 1;
 // The same for row tiles: 512 clocks (256 and 64 measured 7 and 11 % slower
 // sweeps of 512^2: more polls in the way of the publications).
 constexpr int kRowPollDelay = 8;
@@ -268,6 +274,52 @@ struct Fold {
 // SGPR base + VGPR offset addressing instead of flat addressing).
 typedef __attribute__((address_space(1))) unsigned long long gu64;
 
+// Publications as buffer operations at device scope (sc1) on the descriptor's
+// part of the exchange buffer, one aligned 64-bit (value, tag) entry per lane,
+// written and read whole.  A lane that publishes or needs nothing gets kNoHalo
+// as its byte offset: its store is dropped, its load returns 0 without a
+// memory access.  So neither needs a branch, and the loads of all rows are in
+// flight together (under branches the compiler waited for each row's load
+// before it issued the next one).  The offsets fit 32 bits: the tiles of a
+// launch are resident together, and each has two slots of less than 64 KB.
+constexpr unsigned kNoHalo = 0xFFFFFFFFu;
+constexpr int kHaloCache = 16;  // sc1
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t halo_rsrc(unsigned long long *base) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0xFFFFFFF0u, 0x00020000);
+}
+__device__ __forceinline__ void halo_publish(__amdgpu_buffer_rsrc_t h, unsigned ofs, float v, unsigned tag) {
+  __builtin_amdgcn_raw_buffer_store_b64(uint2v{__float_as_uint(v), tag}, h, (int)ofs, 0, kHaloCache);
+}
+__device__ __forceinline__ uint2v halo_read(__amdgpu_buffer_rsrc_t h, unsigned ofs) {
+  asm volatile("" ::: "memory");  // every poll reads again
+  return __builtin_amdgcn_raw_buffer_load_b64(h, (int)ofs, 0, kHaloCache);
+}
+
+// Waits until the entries at ofs[0..N-1] carry `tag` (x holds a first read of
+// them); false after spin_limit more reads.
+template <int N, int REPOLL>
+__device__ __forceinline__ bool halo_wait(__amdgpu_buffer_rsrc_t h, const unsigned (&ofs)[N], uint2v (&x)[N],
+                                          unsigned tag, int spin_limit) {
+  for (int spins = 0;; ++spins) {
+    bool late[N], waiting = false;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      late[k] = ofs[k] != kNoHalo && x[k].y != tag;
+      waiting = waiting || late[k];
+    }
+    if (__ballot(waiting) == 0) return true;
+    if (spins >= spin_limit) return false;
+    __builtin_amdgcn_s_sleep(REPOLL);
+    uint2v y[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) y[k] = halo_read(h, late[k] ? ofs[k] : kNoHalo);
+#pragma unroll
+    for (int k = 0; k < N; ++k) x[k] = late[k] ? y[k] : x[k];
+  }
+}
+
 template <int R, int CT>
 struct Slab {  // one prefetched slice: image rows -1..R, distance rows 0..R-1
   float I[CT][R + 2];
@@ -347,7 +399,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   } else {
     Dd = one;
   }
-  gu64 *halo = (gu64 *)halo_base + Dd.halo0;
+  unsigned long long *const halo = halo_base + Dd.halo0;
   const long long cs = Dd.cs, sA = Dd.sA, sB = Dd.sB;
   const int nA = Dd.nA, nB = Dd.nB, nE = Dd.nE, dir = Dd.dir;
   const float lg = Dd.lg;
@@ -366,14 +418,29 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   const unsigned ec = (unsigned)min(max(e, 0), nE - 1);  // clamped: loads never leave the row
   const unsigned ecb = ec * 4u;                             // its byte offset within a row
   const bool lane_own = (e >= e_own0) && (e < e_own1);
-  const long long tile_slots = (long long)TB * TE;
-  // halo publication slot of this lane (own lanes) and source tile column
-  // of this lane (halo lanes)
-  const int lane_pub = e - e_own0;
+  // Byte offsets (within a parity's slots) of the entry that window row b
+  // publishes, or kNoHalo: own positions within K of a tile edge that has a
+  // neighbour; and of the entry that it reloads, or kNoHalo: non-own
+  // positions within K of the own region (the only ones whose values reach
+  // own positions in K steps), published by the tile that owns them, which
+  // lies across that edge.
+  const int tile_slots = TB * TE;
   const int ote = lane_valid ? (e / TE) : 0;
-  const int oe0 = ote * TE;
-  const int ow = min(nE, oe0 + TE) - oe0;
-  const int lane_src = e - oe0;
+  const int ow = min(nE, ote * TE + TE) - ote * TE;
+  const int lane_dist = max(max(e_own0 - e, e - (e_own1 - 1)), 0);
+  const bool lane_band = (te > 0 && e - e_own0 < K) || (te < nTE - 1 && e_own1 - 1 - e < K);
+  auto publish_ofs = [&](int b) -> unsigned {
+    const bool row_band = (tb > 0 && b - b_own0 < K) || (tb < nTB - 1 && b_own1 - 1 - b < K);
+    if (!(b >= b_own0 && b < b_own1 && lane_own && (row_band || lane_band))) return kNoHalo;
+    return (unsigned)(lt * 2 * tile_slots + (b - b_own0) * (e_own1 - e_own0) + (e - e_own0)) * 8u;
+  };
+  auto reload_ofs = [&](int b) -> unsigned {
+    const bool own = b >= b_own0 && b < b_own1 && lane_own;
+    const int row_dist = max(max(b_own0 - b, b - (b_own1 - 1)), 0);
+    if (b < 0 || b >= nB || !lane_valid || own || max(row_dist, lane_dist) > K) return kNoHalo;
+    const int otb = b / TB;
+    return (unsigned)((otb * nTE + ote) * 2 * tile_slots + (b - otb * TB) * ow + (e - ote * TE)) * 8u;
+  };
 
   // The block loop below advances in groups of P steps and exchanges halos
   // every K steps; it stays within the sweep only when K is a positive
@@ -403,6 +470,12 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     if (w >= NW) {
       constexpr int CR = NWR / kCommWaves;  // window rows per exchange wave
       const int cr0 = (w - NW) * CR;
+      unsigned pub[CR], src[CR];
+#pragma unroll
+      for (int k = 0; k < CR; ++k) {
+        pub[k] = publish_ofs(bw0 + cr0 + k);
+        src[k] = reload_ofs(bw0 + cr0 + k);
+      }
       bool tripped = false;
       for (int blk = 0;; ++blk) {
         for (int st = 0; st < K; ++st) __syncthreads();
@@ -410,61 +483,20 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
         __syncthreads();  // the compute waves' front is in xfront
         const unsigned long long t_in = xhist ? wall_clock64() : 0ull;
         const unsigned tag = tag_base + (unsigned)(blk + 1);
-        const long long hslot = (long long)((blk + 1) & 1) * tile_slots;
-        gu64 *pub = halo + (long long)lt * 2 * tile_slots + hslot;
-        const int own_w = e_own1 - e_own0;
-        const bool lane_band = (te > 0 && e - e_own0 < K) || (te < nTE - 1 && e_own1 - 1 - e < K);
-        const int lane_dist = max(max(e_own0 - e, e - (e_own1 - 1)), 0);
+        const __amdgpu_buffer_rsrc_t h = halo_rsrc(halo + ((blk + 1) & 1) * tile_slots);
 #pragma unroll
-        for (int k = 0; k < CR; ++k) {
-          const int r = cr0 + k;
-          const int b = bw0 + r;
-          const bool row_band = (tb > 0 && b - b_own0 < K) || (tb < nTB - 1 && b_own1 - 1 - b < K);
-          if (b >= b_own0 && b < b_own1 && lane_own && (row_band || lane_band))
-            __hip_atomic_store(pub + (long long)(b - b_own0) * own_w + lane_pub, pack(xfront[r][lane], tag),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        for (int k = 0; k < CR; ++k) halo_publish(h, pub[k], xfront[cr0 + k][lane], tag);
         __builtin_amdgcn_s_sleep(kHaloPollDelay);
-        // whether this lane of window row r needs a neighbour's value, and
-        // where that neighbour publishes it (recomputed rather than held, so
-        // only the 32 loaded words stay live)
-        auto row_need = [&](int r) {
-          const int b = bw0 + r;
-          const bool row_own = b >= b_own0 && b < b_own1;
-          const int row_dist = max(max(b_own0 - b, b - (b_own1 - 1)), 0);
-          return b >= 0 && b < nB && lane_valid && !(row_own && lane_own) && max(row_dist, lane_dist) <= K;
-        };
-        auto row_src = [&](int r) -> const gu64 * {
-          const int bq = min(max(bw0 + r, 0), nB - 1);
-          const int otb = bq / TB;  // uniform
-          return halo + (long long)(otb * nTE + ote) * 2 * tile_slots + hslot + (long long)(bq - otb * TB) * ow +
-                 lane_src;
-        };
-        unsigned long long x[CR];
+        uint2v x[CR];
 #pragma unroll
-        for (int k = 0; k < CR; ++k) {
-          x[k] = (unsigned long long)tag << 32;  // lanes that need nothing count as arrived
-          if (row_need(cr0 + k)) x[k] = __hip_atomic_load(row_src(cr0 + k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        int spins = tripped ? spin_limit : 0;
-        while (true) {
-          bool waiting = false;
-#pragma unroll
-          for (int k = 0; k < CR; ++k) waiting = waiting || (unsigned)(x[k] >> 32) != tag;
-          if (!waiting) break;
-          if (++spins > spin_limit) {
-            __hip_atomic_store(status, FG_EWATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            tripped = true;
-            break;
-          }
-#pragma unroll
-          for (int k = 0; k < CR; ++k)
-            if ((unsigned)(x[k] >> 32) != tag)
-              x[k] = __hip_atomic_load(row_src(cr0 + k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int k = 0; k < CR; ++k) x[k] = halo_read(h, src[k]);
+        if (!halo_wait<CR, kHaloRepollDelay>(h, src, x, tag, tripped ? 0 : spin_limit)) {
+          __hip_atomic_store(status, FG_EWATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          tripped = true;
         }
 #pragma unroll
         for (int k = 0; k < CR; ++k)
-          if (row_need(cr0 + k)) xfront[cr0 + k][lane] = __uint_as_float((unsigned)x[k]);
+          if (src[k] != kNoHalo) xfront[cr0 + k][lane] = __uint_as_float(x[k].x);
         if (xhist && lane == 0) {
           const unsigned long long dt = wall_clock64() - t_in;
           const int bucket = dt ? min(64 - __clzll(dt), kXHistBuckets - 1) : 0;
@@ -761,16 +793,19 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   };
 
   // Publishes the tile's own front values that neighbours read and reloads
-  // the halo positions of the window from the neighbours' publications.
-  //   published: own positions within K of a tile edge that has a neighbour
-  //   reloaded:  non-own window positions within K of the own region (the
-  //              only ones whose values reach own positions in K steps)
-  // A reloaded position's source tile publishes it: it lies within K of that
-  // tile's edge facing this tile.  The prefetch of the next slice is issued
-  // between the halo loads and the wait for them, so that wait does not also
-  // wait for the new prefetch; pending rows are polled together, so one
-  // memory round trip serves all of them.
+  // the halo positions of the window from the neighbours' publications
+  // (publish_ofs, reload_ofs).  Pending rows are polled together, so one
+  // memory round trip serves all of them.  A wave's loads return in order, so
+  // the block's last stores and the prefetch of the next slice follow the
+  // wait: a poll behind them waited for them too (512^3: 702 against 585 us a
+  // sweep with the prefetch before the wait).
   bool wd_tripped = false;
+  unsigned pub[R], src[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    pub[r] = publish_ofs(rb[r + 1]);
+    src[r] = reload_ofs(rb[r + 1]);
+  }
   // COMM: hand the front to the exchange wave and take the halo back from it
   auto exchange_via_comm = [&](int blk, Slab<R, CT> &pf_slab) {
     (void)blk;
@@ -781,15 +816,9 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     advance(cur_pf);
     __syncthreads();  // front visible to the exchange wave
     __syncthreads();  // halo values written by it
-    const int lane_dist = max(max(e_own0 - e, e - (e_own1 - 1)), 0);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int b = rb[r + 1];
-      const bool row_own = b >= b_own0 && b < b_own1;
-      const int row_dist = max(max(b_own0 - b, b - (b_own1 - 1)), 0);
-      const bool need = rvalid[r + 1] && lane_valid && !(row_own && lane_own) && max(row_dist, lane_dist) <= K;
-      if (need) Fd[r] = xfront[w * R + r][lane];
-    }
+    for (int r = 0; r < R; ++r)
+      if (src[r] != kNoHalo) Fd[r] = xfront[w * R + r][lane];
   };
   auto exchange = [&](int blk, Slab<R, CT> &pf_slab) {
     // measurement only (xhist non-null): how long this wave spends in the
@@ -797,74 +826,34 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     // as a histogram of the device's constant-rate clock (log2 buckets)
     const unsigned long long t_in = xhist ? wall_clock64() : 0ull;
     const unsigned tag = tag_base + (unsigned)blk;
-    const long long hslot = (long long)(blk & 1) * tile_slots;
-    gu64 *pub = halo + (long long)lt * 2 * tile_slots + hslot;
-    const int own_w = e_own1 - e_own0;
-    const bool lane_band = (te > 0 && e - e_own0 < K) || (te < nTE - 1 && e_own1 - 1 - e < K);
-    const int lane_dist = max(max(e_own0 - e, e - (e_own1 - 1)), 0);
+    const __amdgpu_buffer_rsrc_t h = halo_rsrc(halo + (blk & 1) * tile_slots);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int b = rb[r + 1];
-      const bool row_band = (tb > 0 && b - b_own0 < K) || (tb < nTB - 1 && b_own1 - 1 - b < K);
-      if (b >= b_own0 && b < b_own1 && lane_own && (row_band || lane_band))
-        __hip_atomic_store(pub + (long long)(b - b_own0) * own_w + lane_pub, pack(Fd[r], tag), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
+    for (int r = 0; r < R; ++r) halo_publish(h, pub[r], Fd[r], tag);
     // XSA: a run completed in this block is stored after the publications (which then leave first) and drains
     // while the wave waits to poll; the halo wait below also waits for it,
     // so every path leaves the exchange with the same loads in flight
     xa_flush();
-    store_last();
     // Neighbours publish at about the same moment; polling right away mostly
-    // finds their values not yet visible and costs a second round trip.
-    // Waiting ~1300 clocks first was measured fastest for 32-row tiles
-    // (16..28 x 64 clocks: 20 best by ~0.2 %, 28 0.5 % slower) and ~770 for
-    // 16-row tiles.
+    // finds their values not yet visible.
     if constexpr (NWR <= 16) __builtin_amdgcn_s_sleep(kHaloPollDelay16);
-    else __builtin_amdgcn_s_sleep(kHaloPollDelay);
-    // Only lanes that need a halo value load (measured faster than letting
-    // every lane load some in-bounds line and selecting afterwards).
-    const gu64 *src[R];
-    bool need[R];
-    unsigned long long x[R];
+    else if (K == P) __builtin_amdgcn_s_sleep(kHaloPollDelay);
+    else __builtin_amdgcn_s_sleep(kHaloPollDelayDeep);
+    uint2v x[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int b = rb[r + 1];
-      const bool row_own = b >= b_own0 && b < b_own1;
-      const int row_dist = max(max(b_own0 - b, b - (b_own1 - 1)), 0);
-      need[r] = rvalid[r + 1] && lane_valid && !(row_own && lane_own) && max(row_dist, lane_dist) <= K;
-      const int bq = min(max(b, 0), nB - 1);
-      const int otb = bq / TB;  // uniform
-      const gu64 *from = halo + (long long)(otb * nTE + ote) * 2 * tile_slots + hslot +
-                         (long long)(bq - otb * TB) * ow + lane_src;
-      src[r] = from;
-      x[r] = 0;
-      if (need[r]) x[r] = __hip_atomic_load(src[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    load_slab(pf_slab, cur_pf, P - 2);
-    advance(cur_pf);
+    for (int r = 0; r < R; ++r) x[r] = halo_read(h, src[r]);
     // after an expiry this wave waits no more: the sweep then finishes
     // (with wrong values, reported through the status word) instead of
     // spending the full limit again at every later exchange
-    int spins = wd_tripped ? spin_limit : 0;
-    while (true) {
-      bool waiting = false;
-#pragma unroll
-      for (int r = 0; r < R; ++r) waiting = waiting || (need[r] && (unsigned)(x[r] >> 32) != tag);
-      if (!waiting) break;
-      if (++spins > spin_limit) {
-        __hip_atomic_store(status, FG_EWATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        wd_tripped = true;
-        break;
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (need[r] && (unsigned)(x[r] >> 32) != tag)
-          x[r] = __hip_atomic_load(src[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!halo_wait<R, (NWR <= 16 ? kHaloRepollDelay16 : kHaloRepollDelay)>(h, src, x, tag, wd_tripped ? 0 : spin_limit)) {
+      __hip_atomic_store(status, FG_EWATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      wd_tripped = true;
     }
+    load_slab(pf_slab, cur_pf, P - 2);
+    advance(cur_pf);
+    store_last();
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      if (need[r]) Fd[r] = __uint_as_float((unsigned)x[r]);
+      if (src[r] != kNoHalo) Fd[r] = __uint_as_float(x[r].x);
     if (xhist && lane == 0) {
       const unsigned long long dt = wall_clock64() - t_in;
       const int bucket = dt ? min(64 - __clzll(dt), kXHistBuckets - 1) : 0;
@@ -876,7 +865,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
   // one (front image).  Afterwards Fr is refilled with the slice of step
   // s + P - 1.
   // j: its number in the block (1..K); the block's last step (no prefetch)
-  // leaves its own-layout stores to the exchange, after the publications.
+  // leaves its own-layout stores to the exchange.
   auto step = [&](Slab<R, CT> &Sl, Slab<R, CT> &Fr, int s, int j, int slot, bool prefetch) {
     // steps past the end of the sweep (the last block is padded to K steps)
     // compute on slices of zeros and store nothing
