@@ -1757,18 +1757,18 @@ constexpr Shape kShapes[] = {{1, 1, kRowHaloStep, kRowHaloStep, false},  {4, 8, 
                              {8, 4, 5, 2, true},   {8, 2, 5, 3, false}};
 constexpr int kNumShapes = 8;
 constexpr int kAutoShape = 5;  // fastest on 512^2 planes: 16 x 2 with the deepest ring that keeps K = 5
-// 16-row windows (8 x 2): with the automatic shape and halo, a pass whose planes (3D,
-// 1-2 channels, general candidate: lamb != 1) all fit the compute units with
-// these tiles at K = 5, and then occupy at least 1.5 x as many of them as
-// with the 32-row windows, runs on them (see Runner::pass_shape): the
-// 32-row windows leave most compute units idle on mid-size planes
-// (128 x 256 x 256: 66-132 tiles) and compute 3.9 x their own tile at
-// K = 10.  Measured on that volume (every pass on 16-row windows): 5.49 ->
-// 4.68 ms (lamb 0.5), 5.52 -> 4.72 ms (lamb 0); lamb 1 unchanged
-// (3.97 / 3.98 ms, bound by the loads rather than the arithmetic); a
-// signed call with every pass on them, including the D pass whose two
-// planes then exceed the device, and batches ran slower (4.18 -> 4.55 ms,
-// 20.7 -> 27.2 ms).
+// 16-row windows (8 x 2, K = 5): with the automatic shape and halo, a pass
+// runs on them when its planes are 3D with 1-2 channels, have several tiles
+// along B, and all their 16-row tiles are resident at one per compute unit
+// (see Runner::pass_shape).  The 32-row windows leave compute units idle on
+// such planes, and a step's time goes with a window's rows.  Planes of one
+// tile along B take a deep halo on the 32-row windows instead, and so do
+// those with lamb = 1 that reach K = 15 there.  Whole calls at iter 2, 16-row
+// against 32-row windows at their best halo, us: 128 x 256 x 256 lamb 1 1651 /
+// 1744, lamb 0.5 1964 / 2358, 2 channels 2373 / 3043; 256^3 lamb 1 2020 / 2134;
+// 128^3 lamb 1 1044 / 1024 (K = 15), lamb 0.5 1226 / 1315; 20 x 120 x 140 lamb 1
+// 780 / 704 (two passes of one tile along B or K = 15).  Passes whose 16-row
+// tiles exceed the device ran slower on them (40 x 400 x 400 lamb 1 2234 / 2019).
 constexpr int kSmallPlaneShape = 7;
 thread_local int g_shape = kAutoShape;
 
@@ -1921,9 +1921,9 @@ const void *pick_row_kernel(int K, bool lamb1, bool fast) {
 
 // The kernel compiled for exactly this (NW, R, P) and channel count, or null.
 // xs selects the output form (0 own layout, 1 B contiguous, 2 A contiguous).
-// B-contiguous kernels exist for the two 5-slice-ring 3D shapes: 8 x 4 with
-// 1-2 channels, 16 x 2 with 1 channel (2 channels would exceed the LDS);
-// A-contiguous ones for both shapes with 1 channel.
+// B-contiguous kernels exist for the 5-slice-ring 3D shapes with 1-2 channels
+// (16 x 2: one; two would exceed the LDS), A-contiguous ones for the same
+// shapes with 1 channel.
 constexpr int kXstMaxC = 2;
 constexpr int kXsaMaxC = 1;
 constexpr int kXsaMaxK = kRunSlots - kRunLen + 1;
@@ -1935,11 +1935,14 @@ const void *pick_kernel(int NW, int R, int P, int C, bool lamb1, bool fast, int 
     if (NW == 8 && R == 4 && P == 5 && C == 1) return pick_variant<8, 4, 5, 1, 1>(lamb1, fast);
     if (NW == 8 && R == 4 && P == 5 && C == 2) return pick_variant<8, 4, 5, 2, 1>(lamb1, fast);
     if (NW == 16 && R == 2 && P == 5 && C == 1) return pick_variant<16, 2, 5, 1, 1>(lamb1, fast);
+    if (NW == 8 && R == 2 && P == 5 && C == 1) return pick_variant<8, 2, 5, 1, 1>(lamb1, fast);
+    if (NW == 8 && R == 2 && P == 5 && C == 2) return pick_variant<8, 2, 5, 2, 1>(lamb1, fast);
     return nullptr;
   }
   if (xs == 2) {
     if (NW == 8 && R == 4 && P == 5 && C == 1) return pick_variant<8, 4, 5, 1, 2>(lamb1, fast);
     if (NW == 16 && R == 2 && P == 5 && C == 1) return pick_variant<16, 2, 5, 1, 2>(lamb1, fast);
+    if (NW == 8 && R == 2 && P == 5 && C == 1) return pick_variant<8, 2, 5, 1, 2>(lamb1, fast);
     return nullptr;
   }
 #define FG_S(nw, r, p, clo, chi) \
@@ -2562,20 +2565,19 @@ struct Runner {
   int pass_shape(const std::vector<Xform *> &active, int pass) {
     if (g_tune.shape != 0 || K != 0 || engine == 0) return g_shape;  // tuned shape or halo
     const std::vector<int> ks = pass_halos(active, pass);  // with the 32-row windows
-    long long t32 = 0, t16 = 0;
+    long long t16 = 0;
     for (size_t i = 0; i < active.size(); ++i) {
       const Xform *x = active[i];
       int nA, nB, nE;
       pass_plane(*x, pass, nA, nB, nE);
       if (nA <= 1) continue;
-      if (x->is2d || nB <= 1 || x->C > 2 || x->lamb1 || ks[i] == 0) return g_shape;
+      if (x->is2d || nB <= 1 || x->C > 2 || ks[i] == 0 || (x->lamb1 && ks[i] >= 15)) return g_shape;
       const Plan a = plan_fixed(nB, nE, ks[i], x->C);
       const Plan b = plan_fixed(nB, nE, 5, x->C, kSmallPlaneShape);
-      if (!a.ok || !b.ok) return g_shape;
-      t32 += (long long)a.nTB * a.nTE;
+      if (!a.ok || !b.ok || a.nTB == 1) return g_shape;
       t16 += (long long)b.nTB * b.nTE;
     }
-    return (t16 > 0 && t16 <= dev.cus && 2 * t16 >= 3 * t32) ? kSmallPlaneShape : g_shape;
+    return (t16 > 0 && t16 <= dev.cus) ? kSmallPlaneShape : g_shape;
   }
 
   // Record one pass (forward then backward) for the active transforms.
