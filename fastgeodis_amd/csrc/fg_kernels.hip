@@ -1360,6 +1360,177 @@ __global__ __launch_bounds__(kRowThreads)
 }
 
 // ---------------------------------------------------------------------------
+// Small 2D images: a whole transform in one workgroup
+// ---------------------------------------------------------------------------
+
+// One transform, every sweep of every iteration, with image and distance in
+// LDS.
+struct SmallDesc {
+  const float *img;  // (C, H, W)
+  const float *src;  // mask (init_mode 1: v*m, 2: v*(1-m)) or initial distance (0)
+  float *out;        // (H, W), or (W, H) with `flip`
+  int C, H, W, iters;
+  int init_mode, flip;
+  float v, lg, e1s, e1c;  // e1s: step to a side neighbour of the previous line, e1c: to the middle one
+};
+
+// The transforms of one call (signed 2, GSF 4) travel in the kernel's
+// arguments: a descriptor copy of its own would cost ~15 us on the stream.
+constexpr int kSmallByValue = 4;
+struct SmallDescs {
+  SmallDesc d[kSmallByValue];
+};
+
+constexpr int kSmallWaves = 4, kSmallHalo = 16, kSmallOwn = 64 - 2 * kSmallHalo;
+constexpr int kSmallSide = kSmallWaves * kSmallOwn;  // longest side
+constexpr int kSmallAhead = 4;                       // lines read ahead
+// Floats per element in LDS: the distance and up to 1 or 3 image channels.
+constexpr int small_element(int C) { return C == 1 ? 2 : 4; }
+// Floats before and after the image that reads ahead of the last line touch.
+constexpr int small_guard(int C, int W) { return kSmallAhead * (W | 1) * small_element(C); }
+// LDS of an H x W image: rows of odd pitch, so that both lines of consecutive
+// elements and columns spread over the banks; the guards; one word per thread
+// for the lanes that store nothing.
+constexpr size_t small_lds(int C, int H, int W) {
+  return ((size_t)H * (W | 1) * small_element(C) + 2 * small_guard(C, W) + kSmallWaves * 64) * sizeof(float);
+}
+
+template <int EL>
+struct SmallElement;
+template <>
+struct SmallElement<2> { typedef float2 type; };
+template <>
+struct SmallElement<4> { typedef float4 type; };
+
+// A call on a small image is launches: at 64^2 a sweep's 63 steps take ~2 us
+// of the ~8 us that its launch, first loads and exchanges cost.  Here one
+// launch does everything: the image and the distance sit in LDS, a line of up
+// to 64 elements is one wave's, a longer one is split over up to four waves
+// with 32 own lanes each and 16 lanes of halo to either side, which are read
+// back from the lines in LDS every 16 steps behind a barrier.  64^2, one
+// channel, iter 2: 73 -> 33 us a call; 128^2 98 -> 78 us.
+template <int CT, bool LAMB1, bool FAST>
+__global__ __launch_bounds__(kSmallWaves * 64) void small_call_kernel(const SmallDesc *__restrict__ descs,
+                                                                      SmallDescs few) {
+  constexpr int EL = CT == 1 ? 2 : 4;
+  typedef typename SmallElement<EL>::type Element;
+  extern __shared__ __align__(16) float small_mem[];
+  SmallDesc S;
+  if (descs) {
+    S = descs[blockIdx.x];
+  } else {
+    S = few.d[0];
+#pragma unroll
+    for (int k = 1; k < kSmallByValue; ++k)
+      if ((int)blockIdx.x == k) S = few.d[k];
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int H = S.H, W = S.W, pitch = W | 1;
+  const long long N = (long long)H * W;
+  const int guard = small_guard(CT, W);
+  float *const mem = small_mem + guard;
+  for (int h = wave; h < H; h += kSmallWaves)
+    for (int x = lane; x < W; x += 64) {
+      const int k = h * W + x;
+      const float m = S.src[k], t = 1.0f - m;
+      float *el = mem + (h * pitch + x) * EL;
+      el[0] = S.init_mode == 0 ? m : S.v * (S.init_mode == 2 ? t : m);
+#pragma unroll
+      for (int c = 0; c < CT; ++c) el[1 + c] = S.img[c * N + k];
+    }
+  __syncthreads();
+
+  const float e1[9] = {0.f, 0.f, 0.f, S.e1s, S.e1c, S.e1s, 0.f, 0.f, 0.f};
+  const float lg = S.lg;
+  for (int sweep = 0; sweep < 4 * S.iters; ++sweep) {
+    const bool rows = (sweep & 2) == 0;
+    const int dir = (sweep & 1) ? -1 : 1;
+    const int nA = rows ? H : W, nE = rows ? W : H;
+    const int sA = (rows ? pitch : 1) * EL, sE = (rows ? 1 : pitch) * EL;  // floats
+    const int nsteps = nA - 1, a0 = dir > 0 ? 0 : nA - 1;
+    const bool split = nE > 64;
+    const int e = split ? wave * kSmallOwn - kSmallHalo + lane : lane;
+    const bool own = e >= 0 && e < nE && (!split || (lane >= kSmallHalo && lane < 64 - kSmallHalo));
+    const bool has_left = e > 0, has_right = e < nE - 1;
+    const bool active = wave == 0 || (split && wave * kSmallOwn < nE);
+    // read position kSmallAhead lines ahead of the step, write position; lanes
+    // that store nothing write a word of their own
+    const float *rp = mem + a0 * sA + min(max(e, 0), nE - 1) * sE;
+    float *wp = own ? mem + (a0 + dir) * sA + e * sE : small_mem + H * pitch * EL + 2 * guard + threadIdx.x;
+    const int rs = dir * sA, ws = own ? rs : 0;
+    float F = 0.f, Iq[CT];
+    Element q[kSmallAhead];
+    auto read = [&]() {
+      const Element x = *reinterpret_cast<const Element *>(rp);
+      rp += rs;
+      return x;
+    };
+    if (active) {
+      const Element f = read();
+      const float *pf = reinterpret_cast<const float *>(&f);
+      F = pf[0];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) Iq[c] = pf[1 + c];
+#pragma unroll
+      for (int k = 0; k < kSmallAhead; ++k) q[k] = read();
+    }
+    auto step = [&](Element &x) {
+      const float *pq = reinterpret_cast<const float *>(&x);
+      const float dinit = pq[0];
+      float In[CT];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) In[c] = pq[1 + c];
+      x = read();
+      float t[3];
+      candidates_row<1, CT, LAMB1>(t, F, Iq, In, e1, lg);
+      t[0] = has_left ? t[0] : kInf;
+      t[2] = has_right ? t[2] : kInf;
+      if constexpr (FAST) {
+        const float m = fminf(fminf(t[0], t[1]), t[2]);
+        F = (m < dinit) ? m : dinit;
+      } else {
+        F = dinit;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) F = (t[i] < F) ? t[i] : F;
+      }
+#pragma unroll
+      for (int c = 0; c < CT; ++c) Iq[c] = In[c];
+      *wp = F;
+      wp += ws;
+    };
+    for (int s0 = 0; s0 < nsteps; s0 += kSmallHalo) {
+      if (split && s0 > 0) {
+        __syncthreads();  // every wave's own part of the last line is in LDS
+        if (active) {
+          const float x = rp[-(1 + kSmallAhead) * rs];
+          F = own ? F : x;
+        }
+      }
+      if (active) {
+        const int n = min(kSmallHalo, nsteps - s0);
+        int j = 0;
+        for (; j + kSmallAhead <= n; j += kSmallAhead) {
+#pragma unroll
+          for (int k = 0; k < kSmallAhead; ++k) step(q[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kSmallAhead - 1; ++k)
+          if (j + k < n) step(q[k]);
+      }
+    }
+    __syncthreads();
+  }
+
+  if (!S.flip) {
+    for (int h = wave; h < H; h += kSmallWaves)
+      for (int x = lane; x < W; x += 64) S.out[h * W + x] = mem[(h * pitch + x) * EL];
+  } else {
+    for (int x = wave; x < W; x += kSmallWaves)
+      for (int h = lane; h < H; h += 64) S.out[x * H + h] = mem[(h * pitch + x) * EL];
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Per-slice engine: one launch updates one slice from the previous one.
 // Visits candidates in the reference order with the reference's min rule.
 // ---------------------------------------------------------------------------
@@ -1715,6 +1886,7 @@ struct Xform {
   bool lamb1, fast;
   int iters;
   int it = 0;  // the iteration being recorded
+  bool small = false;  // runs in one workgroup (small_call_kernel)
   bool xst;  // this iteration's H-backward sweep writes dT directly (no transpose before the W pass)
   bool xsa = false;  // this iteration's W-backward sweep writes d directly (no transpose after the W pass)
   // The first sweep initialises the distance from the mask (init_mode 1: v*m,
@@ -1919,6 +2091,21 @@ const void *pick_row_kernel(int K, bool lamb1, bool fast) {
   }
 }
 
+template <int CT>
+const void *pick_small_variant(bool lamb1, bool fast) {
+  if (lamb1) return reinterpret_cast<const void *>(&small_call_kernel<CT, true, true>);
+  return fast ? reinterpret_cast<const void *>(&small_call_kernel<CT, false, true>)
+              : reinterpret_cast<const void *>(&small_call_kernel<CT, false, false>);
+}
+const void *pick_small_kernel(int C, bool lamb1, bool fast) {
+  switch (C) {
+    case 1: return pick_small_variant<1>(lamb1, fast);
+    case 2: return pick_small_variant<2>(lamb1, fast);
+    case 3: return pick_small_variant<3>(lamb1, fast);
+    default: return nullptr;
+  }
+}
+
 // The kernel compiled for exactly this (NW, R, P) and channel count, or null.
 // xs selects the output form (0 own layout, 1 B contiguous, 2 A contiguous).
 // B-contiguous kernels exist for the 5-slice-ring 3D shapes with 1-2 channels
@@ -1977,7 +2164,9 @@ struct Carver {
 // Recorded launch.  Descriptor arrays live in one host blob that is copied to
 // the workspace once per call, before any launch is issued.
 struct Cmd {
-  enum Type { TILED, SLICE, XPOSE, EW } type;
+  enum Type { TILED, SLICE, XPOSE, EW, SMALL } type;
+  size_t lds = 0;  // dynamic LDS bytes
+  SmallDescs small_few{};
   const void *kern = nullptr;
   int grid = 0, block = 0;
   size_t off = 0;  // descriptor offset in the blob
@@ -2713,13 +2902,69 @@ struct Runner {
     }
   }
 
+  // The small transforms of a run: one workgroup each, one launch per kernel
+  // and LDS size class, then the epilogues of their groups.
+  int record_small(std::vector<Xform> &xs) {
+    struct Launch { const void *kern; size_t lds; std::vector<SmallDesc> descs; };
+    std::vector<Launch> launches;
+    std::vector<Xform *> mine;
+    for (auto &x : xs) {
+      if (!x.small) continue;
+      const bool flip = x.fin_member || x.fin_kind != XK_COPY;  // an epilogue reads the W pass layout
+      SmallDesc d{};
+      d.img = x.img;
+      d.src = x.init_mode ? x.init_src : x.d;
+      d.out = flip ? x.dT : x.d;
+      d.C = x.C; d.H = x.H; d.W = x.W; d.iters = x.iters;
+      d.init_mode = x.init_mode;
+      d.flip = flip;
+      d.v = x.init_v;
+      d.lg = x.lg;
+      d.e1s = x.e1[1][3];
+      d.e1c = x.e1[1][4];
+      const void *kern = pick_small_kernel(x.C, x.lamb1, x.fast);
+      if (!kern) return fail(FG_EINVAL, "internal: no kernel for a small image");
+      const size_t lds = small_lds(x.C, x.H, x.W);
+      // (workgroups of one launch reserve the same LDS: a class per 32 KB)
+      auto l = std::find_if(launches.begin(), launches.end(),
+                            [&](const Launch &q) { return q.kern == kern && (q.lds >> 15) == (lds >> 15); });
+      if (l == launches.end()) l = launches.insert(launches.end(), {kern, lds, {}});
+      l->lds = std::max(l->lds, lds);
+      l->descs.push_back(d);
+      x.it = x.iters - 1;
+      x.xsa = !flip;
+      mine.push_back(&x);
+    }
+    for (auto &l : launches) {
+      Cmd c;
+      c.type = Cmd::SMALL;
+      c.kern = l.kern;
+      c.lds = l.lds;
+      c.grid = c.ndesc = (int)l.descs.size();
+      c.block = kSmallWaves * 64;
+      if (c.ndesc <= kSmallByValue) {
+        c.by_value = true;
+        std::copy(l.descs.begin(), l.descs.end(), c.small_few.d);
+      } else {
+        c.off = rec.put(l.descs.data(), l.descs.size() * sizeof(SmallDesc));
+      }
+      rec.cmds.push_back(c);
+    }
+    std::vector<XposeDesc> back;
+    w_pass_back(mine, back);
+    record_xpose(back);
+    return FG_OK;
+  }
+
   int record_run(std::vector<Xform> &xs) {
+    if (const int rc = record_small(xs)) return rc;
     int max_it = 0;
-    for (auto &x : xs) max_it = std::max(max_it, x.iters);
+    for (auto &x : xs)
+      if (!x.small) max_it = std::max(max_it, x.iters);
     for (int it = 0; it < max_it; ++it) {
       std::vector<Xform *> active;
       for (auto &x : xs)
-        if (x.iters > it) {
+        if (!x.small && x.iters > it) {
           x.it = it;
           active.push_back(&x);
         }
@@ -2828,6 +3073,11 @@ struct Runner {
           a = {(void *)&v.dp, &v.ndesc, (void *)&c.xpose1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
           funcs[i] = reinterpret_cast<const void *>(&xpose_kernel);
           break;
+        case Cmd::SMALL:
+          v.dp = c.by_value ? nullptr : blob_dev + c.off;
+          a = {(void *)&v.dp, (void *)&c.small_few, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+          funcs[i] = c.kern;
+          break;
         case Cmd::EW:
           v.dp = c.by_value ? nullptr : blob_dev + c.off;
           a = {(void *)&v.dp, &v.ndesc, (void *)&c.ew1, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -2840,7 +3090,7 @@ struct Runner {
       p.func = const_cast<void *>(funcs[i]);
       p.gridDim = dim3(rec.cmds[i].grid);
       p.blockDim = dim3(rec.cmds[i].block);
-      p.sharedMemBytes = 0;
+      p.sharedMemBytes = (unsigned)rec.cmds[i].lds;
       p.kernelParams = args[i].data();
       p.extra = nullptr;
       return p;
@@ -2855,6 +3105,7 @@ struct Runner {
         mix((uint64_t)(uintptr_t)funcs[i]);
         mix((uint64_t)rec.cmds[i].grid);
         mix((uint64_t)rec.cmds[i].block);
+        mix((uint64_t)rec.cmds[i].lds);
       }
       GraphEntry *e = nullptr;
       {
@@ -2930,7 +3181,7 @@ struct Runner {
         FG_HIP(hipEventCreate(&pr.stop));
         FG_HIP(hipEventRecord(pr.start, stream));
       }
-      FG_HIP(hipLaunchKernel(funcs[i], dim3(c.grid), dim3(c.block), args[i].data(), 0, stream));
+      FG_HIP(hipLaunchKernel(funcs[i], dim3(c.grid), dim3(c.block), args[i].data(), c.lds, stream));
       if (prof) {
         FG_HIP(hipEventRecord(pr.stop, stream));
         pr.bytes = c.alg_bytes;
@@ -2990,6 +3241,23 @@ void make_xform(const OpSpec &o, float lg, float le, Xform &x) {
 
 long long vox(const OpSpec &o) { return (long long)o.D * o.H * o.W; }
 
+// Whether an op's transforms can run in one workgroup each: 2D, one channel with
+// sides up to kSmallSide or 2-3 channels with sides up to 64, the tiled engine
+// and no requested halo depth or workgroup cap.  The one front wave of
+// small_call_kernel takes longer per step than row_sweep_kernel's (~60 ns with
+// one channel, ~110 with 3, against ~42) but nothing per launch.  us a call at
+// iter 2, this kernel / one launch per sweep: 64^2 33 / 73, 128^2 78 / 98,
+// 128 x 100 lamb 0.5 87 / 96; 3 channels lamb 0.5: 64^2 57 / 77, 90^2 92 / 82.
+bool small_op(const OpSpec &o) {
+  const int side = std::max(o.H, o.W);
+  return o.is2d && o.iters > 0 && side <= (o.C == 1 ? kSmallSide : 64) && o.C <= 3 && g_tune.engine != 0 &&
+         g_tune.halo == 0 && g_tune.max_groups == 0 && small_lds(o.C, o.H, o.W) <= (160u << 10);
+}
+// They do when all ops of the call can: beside larger ones they share those
+// launches at no cost of their own (a batch of 48 images and 8 volumes: 4735
+// us, 4896 with its small images in launches of their own).
+bool small_ops(const std::vector<OpSpec> &ops) { return std::all_of(ops.begin(), ops.end(), small_op); }
+
 int n_dist(int op) { return op == FG_OP_UNSIGNED ? 1 : (op == FG_OP_SIGNED ? 2 : 4); }
 
 size_t halo_entries_for(const std::vector<OpSpec> &ops, int K) {
@@ -3031,6 +3299,7 @@ size_t blob_bytes_for(const std::vector<OpSpec> &ops) {
   bytes += nsweep * (ntrans * sizeof(SweepDesc) + 256) * 2;
   bytes += (4 * sets + 2) * (ntrans * sizeof(XposeDesc) + 256) + (ops.size() * sizeof(XposeDesc) + 256);
   bytes += 8 * (ops.size() * sizeof(EwDesc) + 256);
+  bytes += 2 * (ntrans * (sizeof(SmallDesc) + 256));
   return bytes + 4096;
 }
 
@@ -3124,14 +3393,15 @@ int run_ops(std::vector<OpSpec> &ops, void *ws, size_t wsb, hipStream_t stream, 
   if (!cv.fits()) return fail(FG_EWORKSPACE, "workspace too small");
 
   // the halo tags start from zero on every call
-  run.record_zero_halo();
+  const bool small = small_ops(ops);
+  if (!small) run.record_zero_halo();
 
   // image transposes (once per op)
   {
     std::vector<XposeDesc> xs;
     for (size_t i = 0; i < ops.size(); ++i) {
       const OpSpec &o = ops[i];
-      if (o.imageT) continue;  // the caller keeps the transposed image
+      if (o.imageT || small) continue;  // the caller keeps the transposed image; small ones need none
       if (o.is2d) xs.push_back(Runner::xd(o.image, bufs[i].imgT, o.C, o.H, 1, o.W));
       else xs.push_back(Runner::xd(o.image, bufs[i].imgT, o.C, o.D, o.H, o.W));
     }
@@ -3186,8 +3456,9 @@ int run_ops(std::vector<OpSpec> &ops, void *ws, size_t wsb, hipStream_t stream, 
       c.nelem = N * (o.Cm - 1);
       chans.push_back(c);
     }
-    bool tiled = false;
-    if ((rc = run.first_sweep_tiled(xs[j0], tiled))) return rc;
+    for (int k = 0; k < nd; ++k) xs[j0 + k].small = small;
+    bool tiled = xs[j0].small;
+    if (!tiled && (rc = run.first_sweep_tiled(xs[j0], tiled))) return rc;
     if (tiled) {
       for (int k = 0; k < nd; ++k) {
         xs[j0 + k].init_mode = (k == 0) ? 1 : 2;
@@ -3257,6 +3528,7 @@ int run_ops(std::vector<OpSpec> &ops, void *ws, size_t wsb, hipStream_t stream, 
         x.imgT = bufs[i].imgT;
         x.d = bufs[i].dist[k];
         x.dT = bufs[i].dT[k];
+        x.small = small;
         xs2.push_back(x);
       }
       if (fused[i]) {

@@ -79,3 +79,34 @@ def test_channels_share_a_launch(depth):
         wants.append(want)
     for got, want in zip(FG.geodesic_batch(insts), wants):
         assert equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("C,H,W", [(1, 1, 1), (1, 2, 3), (1, 63, 64), (1, 64, 65), (1, 65, 97), (1, 96, 128),
+                                   (1, 128, 127), (1, 129, 64), (2, 64, 63), (3, 64, 64), (3, 65, 64)])
+@pytest.mark.parametrize("lamb", [1.0, 0.5, 1.5])
+def test_small_images(device, C, H, W, lamb):
+    """Whole transforms in one workgroup, at the sizes around its limits and
+    line splits; and several in one call beside images too large for it."""
+    rng = np.random.default_rng(H * 131 + W)
+    for special in (False, True):
+        img, m = make(rng, C, H, W, special)
+        ti, tm = torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda()
+        print(f"small C={C} {H}x{W} lamb={lamb} special={special}", flush=True)
+        with np.errstate(all="ignore"):
+            for it in (0, 1, 3):
+                assert equal(FG.generalised_geodesic2d(ti, tm, 1e10, lamb, it).cpu().numpy(),
+                             oracle.py_geodesic2d(img, m, 1e10, lamb, it))
+    mask = (rng.random((1, 2, H, W)) > 0.5).astype(np.float32)
+    img, _ = make(rng, C, H, W)
+    ti, tm = torch.from_numpy(img).cuda(), torch.from_numpy(mask).cuda()
+    assert equal(FG.signed_generalised_geodesic2d(ti, tm, 1e3, lamb, 2).cpu().numpy(),
+                 oracle.py_signed_geodesic2d(img, mask, 1e3, lamb, 2))
+    want = oracle.py_gsf2d(img, mask, 0.1, 1e3, lamb, 2)
+    assert equal(FG.GSF2d(ti, tm, 0.1, 1e3, lamb, 2).cpu().numpy(), want)
+    big, bm = make(rng, 1, 150, 70)
+    insts = [FG.Instance(torch.from_numpy(big).cuda(), torch.from_numpy(bm).cuda(), 1e10, lamb, iter=2)]
+    insts += [FG.Instance(ti, tm, 1e3, lamb, iter=2, op="gsf", theta=0.1) for _ in range(3)]
+    assert all(equal(g.cpu().numpy(), want) for g in FG.geodesic_batch(insts[1:]))
+    got = FG.geodesic_batch(insts)
+    assert equal(got[0].cpu().numpy(), oracle.py_geodesic2d(big, bm, 1e10, lamb, 2))
+    assert all(equal(g.cpu().numpy(), want) for g in got[1:])
