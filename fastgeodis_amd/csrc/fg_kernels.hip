@@ -213,22 +213,40 @@ __device__ __forceinline__ float candidate(float dq, const float (&Iq)[CT], cons
   // shift folds into v_sub_f32_dpp without commuting
   const float l =
       absdiff_sum<I, J, 1, CT>(fabsf(shiftE<J, 1 + I * 16 + J * 4, (I & 1) != 0>(Iq[0]) - In[0]), Iq, In);
-  const float ds = shiftE<J, 64 + I * 4 + J, (I & 1) != 0>(dq);
   if constexpr (LAMB1) {
     // l_grad == 1 and l_eucl*LD == +0: fl(1*l) == l and dropping "+ 0" is exact here
-    return ds + l;
+    return shiftE<J, 64 + I * 4 + J, (I & 1) != 0>(dq) + l;
   } else {
-    return (ds + e1) + lg * l;
+    // the step is added before the shift, so that the candidates of several
+    // new elements share the sums of a front element: with the table's equal
+    // entries (step_of) 12 additions per two rows instead of 18
+    return shiftE<J, 64 + I * 4 + J, (I & 1) != 0>(dq + e1) + lg * l;
   }
+}
+
+// The table entry of a candidate: steps to opposite neighbours have the same
+// length (and bits), so each is taken from the first of its kind.
+template <int I, int J>
+__device__ __forceinline__ float step_of(const float (&e1)[9]) {
+  return e1[(I == 2 ? 0 : I) * 3 + (J == 2 ? 0 : J)];
 }
 
 // The three candidates from front row I (its distance dq and image Iq).
 template <int I, int CT, bool LAMB1>
 __device__ __forceinline__ void candidates_row(float (&c)[3], float dq, const float (&Iq)[CT],
                                                const float (&In)[CT], const float (&e1)[9], float lg) {
-  c[0] = candidate<I, 0, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 0], lg);
-  c[1] = candidate<I, 1, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 1], lg);
-  c[2] = candidate<I, 2, CT, LAMB1>(dq, Iq, In, e1[I * 3 + 2], lg);
+  c[0] = candidate<I, 0, CT, LAMB1>(dq, Iq, In, step_of<I, 0>(e1), lg);
+  c[1] = candidate<I, 1, CT, LAMB1>(dq, Iq, In, step_of<I, 1>(e1), lg);
+  c[2] = candidate<I, 2, CT, LAMB1>(dq, Iq, In, step_of<I, 2>(e1), lg);
+}
+
+// v_min3_f32 of quiet operands (results of arithmetic).  Where one comes from
+// another basic block, the compiler would quiet it first and fall back to
+// two-operand minima: six more instructions per two rows behind the barrier.
+__device__ __forceinline__ float min3(float a, float b, float c) {
+  float r;
+  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
 }
 
 // The nine candidates of one row element in the order they become available:
@@ -249,8 +267,7 @@ struct Fold {
         m = fminf(fminf(m, t[0]), t[1]);
         left = t[2];
       } else {
-        m = fminf(fminf(m, left), t[0]);
-        m = fminf(fminf(m, t[1]), t[2]);
+        m = min3(min3(m, left, t[0]), t[1], t[2]);
       }
       ++n;
     } else {
