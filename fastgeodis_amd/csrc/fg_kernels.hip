@@ -2004,15 +2004,20 @@ Plan plan_fixed(int nB, int nE, int Kreq, int C, int shape = -1) {
 
 // Plan of one sweep plane.  Kreq > 0: that halo depth, rounded up to a
 // multiple of the slab ring (a row whose tiles would not all be resident at
-// that depth takes the deepest at which they are).  Kreq == 0 (automatic):
+// that depth takes the deepest at which they are, in a 3D volume one whose
+// entries fit the exchange buffer of the requested depth).  Kreq == 0 (automatic):
 // the deepest halo (fewest exchanges) whose tiles still fit one per compute
 // unit (rows: row_groups_per_cu), as every tile waits for its neighbours at
 // each exchange; if even the shallowest halo needs more tiles, that one.
-Plan plan_plane(int nB, int nE, int Kreq, int C, int tile_budget) {
+Plan plan_plane(int nB, int nE, int Kreq, int C, int tile_budget, bool is2d) {
   auto budget = [&](int K) { return nB == 1 ? tile_budget * row_groups_per_cu(K) : tile_budget; };
   if (Kreq > 0) {
-    Plan p = plan_fixed(nB, nE, Kreq, C);
-    while (nB == 1 && p.nTE > 2 * tile_budget && p.K > p.P) p = plan_fixed(nB, nE, p.K - p.P, C);
+    const Plan p = plan_fixed(nB, nE, Kreq, C);
+    if (nB > 1 || p.nTE <= 2 * tile_budget) return p;
+    for (int K = p.K - p.P; K > 0; K -= p.P) {
+      const Plan q = plan_fixed(nB, nE, K, C);
+      if ((q.nTE <= 2 * tile_budget || K == p.P) && (is2d || q.nTE * q.TE <= p.nTE * p.TE)) return q;
+    }
     return p;
   }
   const Plan first = plan_fixed(nB, nE, 1, C);
@@ -2521,7 +2526,7 @@ struct Runner {
     int nA, nB, nE;
     pass_plane(x, 1, nA, nB, nE);
     if (nA <= 1 || nB <= 1) return false;
-    const Plan p = plan_plane(nB, nE, K, x.C, dev.cus);
+    const Plan p = plan_plane(nB, nE, K, x.C, dev.cus, x.is2d);
     if (!p.ok || !pick_kernel(p.NW, p.R, p.P, x.C, x.lamb1, x.fast, 1, false, p.comm)) return false;
     if ((long long)x.D * x.H * x.W * 4 >= 0xFFFFFFF0ll) return false;
     return slice_offsets_fit(x, 1);
@@ -2704,7 +2709,7 @@ struct Runner {
     int nA, nB, nE;
     pass_plane(x, pass, nA, nB, nE);
     if (nA <= 1 || engine == 0 || x.C > 4) return false;
-    return plan_plane(nB, nE, K, x.C, dev.cus).ok && slice_offsets_fit(x, pass);
+    return plan_plane(nB, nE, K, x.C, dev.cus, x.is2d).ok && slice_offsets_fit(x, pass);
   }
 
   // Halo depth of each transform's plane in this pass.  Requested depths
@@ -2724,7 +2729,7 @@ struct Runner {
       int nA, nB, nE;
       pass_plane(*active[i], pass, nA, nB, nE);
       if (!tiled_eligible(*active[i], pass)) continue;
-      ks[i] = plan_plane(nB, nE, K, active[i]->C, dev.cus).K;
+      ks[i] = plan_plane(nB, nE, K, active[i]->C, dev.cus, active[i]->is2d).K;
       if (K == 0) (nB > 1 ? planes : rows).push_back((int)i);
     }
     if (rows.size() > 1) share_halo(active, pass, rows, ks);
@@ -3286,7 +3291,7 @@ size_t halo_entries_for(const std::vector<OpSpec> &ops, int K) {
     for (int p = 0; p < 3; ++p) {
       int nA, nB, nE;
       pass_plane(x, p, nA, nB, nE);
-      const bool any = K <= 0 || nB == 1;  // depths the plan may take
+      const bool any = K <= 0 || o.is2d;  // depths the plan may take
       for (int k = (any ? 1 : K); k <= (any ? kMaxK : K); ++k) {
         for (int sh : {g_shape, (g_tune.shape == 0 && K <= 0) ? kSmallPlaneShape : g_shape}) {
           Plan pl = plan_fixed(nB, nE, k, o.C, sh);
@@ -3304,10 +3309,11 @@ size_t halo_entries_for(const std::vector<OpSpec> &ops, int K) {
 // once, and the active set of transforms changes at most once per distinct
 // iteration count.
 size_t blob_bytes_for(const std::vector<OpSpec> &ops) {
-  size_t ntrans = 0;
+  size_t ntrans = 0, n2d = 0;
   std::vector<int> its;
   for (auto &o : ops) {
     ntrans += n_dist(o.op);
+    if (o.is2d) n2d += n_dist(o.op);
     if (std::find(its.begin(), its.end(), o.iters) == its.end()) its.push_back(o.iters);
   }
   const size_t sets = its.size() + 1;
@@ -3316,7 +3322,7 @@ size_t blob_bytes_for(const std::vector<OpSpec> &ops) {
   bytes += nsweep * (ntrans * sizeof(SweepDesc) + 256) * 2;
   bytes += (4 * sets + 2) * (ntrans * sizeof(XposeDesc) + 256) + (ops.size() * sizeof(XposeDesc) + 256);
   bytes += 8 * (ops.size() * sizeof(EwDesc) + 256);
-  bytes += 2 * (ntrans * (sizeof(SmallDesc) + 256));
+  bytes += 2 * (n2d * (sizeof(SmallDesc) + 256));
   return bytes + 4096;
 }
 
