@@ -1049,7 +1049,7 @@ constexpr int row_groups_per_cu(int K) { return K >= 30 ? 1 : K >= 24 ? 2 : K >=
 
 // Everything of a row tile that both kinds of wave use.
 struct RowTile {
-  int lane, e, ew0, e_own0, e_own1;
+  int te, lane, e, ew0, e_own0, e_own1;
   bool lane_valid, lane_own;
   int nA, dir, a_first, nsteps, nblocks;
   unsigned stride4;     // bytes of a slice (a row of lanes)
@@ -1057,6 +1057,29 @@ struct RowTile {
   unsigned range;       // bytes of the array
   unsigned lofs;        // this lane's byte offset in a slice, clamped into it
 };
+
+__device__ __forceinline__ RowTile row_tile(const SweepDesc &Dd, int te, int K) {
+  const int nTE = Dd.nTE, TE = Dd.TE, nE = Dd.nE;
+  RowTile T;
+  T.te = te;
+  T.lane = threadIdx.x & 63;
+  T.e_own0 = te * TE;
+  T.e_own1 = min(nE, T.e_own0 + TE);
+  T.ew0 = (nTE > 1) ? T.e_own0 - K : -1;
+  T.e = T.ew0 + T.lane;
+  T.lane_valid = T.e >= 0 && T.e < nE;
+  T.lane_own = T.e >= T.e_own0 && T.e < T.e_own1;
+  T.nA = Dd.nA;
+  T.dir = Dd.dir;
+  T.nsteps = Dd.nA - 1;
+  T.nblocks = (T.nsteps + K - 1) / K;
+  T.a_first = Dd.dir > 0 ? 1 : Dd.nA - 2;
+  T.stride4 = (unsigned)Dd.sA * 4u;
+  T.dstride4 = (unsigned)Dd.dir * T.stride4;
+  T.range = (unsigned)((long long)Dd.nA * Dd.sA * 4);
+  T.lofs = (unsigned)min(max(T.e, 0), nE - 1) * 4u;
+  return T;
+}
 
 // Byte offset of slice a of the sweep's arrays.  Slices before the first or
 // past the last one give offsets at or beyond the array's range (the host
@@ -1267,25 +1290,8 @@ __global__ __launch_bounds__(kRowThreads)
     if (threadIdx.x == 0) __hip_atomic_store(status, FG_EINVAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return;
   }
-  const int nTE = Dd.nTE, TE = Dd.TE, nE = Dd.nE;
-  const int te = tile - Dd.tile0;
-  RowTile T;
-  T.lane = threadIdx.x & 63;
-  T.e_own0 = te * TE;
-  T.e_own1 = min(nE, T.e_own0 + TE);
-  T.ew0 = (nTE > 1) ? T.e_own0 - K : -1;
-  T.e = T.ew0 + T.lane;
-  T.lane_valid = T.e >= 0 && T.e < nE;
-  T.lane_own = T.e >= T.e_own0 && T.e < T.e_own1;
-  T.nA = Dd.nA;
-  T.dir = Dd.dir;
-  T.nsteps = Dd.nA - 1;
-  T.nblocks = (T.nsteps + K - 1) / K;
-  T.a_first = Dd.dir > 0 ? 1 : Dd.nA - 2;
-  T.stride4 = (unsigned)Dd.sA * 4u;
-  T.dstride4 = (unsigned)Dd.dir * T.stride4;
-  T.range = (unsigned)((long long)Dd.nA * Dd.sA * 4);
-  T.lofs = (unsigned)min(max(T.e, 0), nE - 1) * 4u;
+  const RowTile T = row_tile(Dd, tile - Dd.tile0, K);
+  const int nTE = Dd.nTE, TE = Dd.TE, te = T.te;
   if (T.nsteps <= 0) return;
 
   if (w > 0) {
@@ -1385,6 +1391,170 @@ __global__ __launch_bounds__(kRowThreads)
       }
     }
     __syncthreads();
+  }
+  if (xhist) {
+    __syncthreads();
+    if (threadIdx.x < kXHistBuckets && xhist_wg[threadIdx.x]) atomicAdd(xhist + threadIdx.x, xhist_wg[threadIdx.x]);
+  }
+}
+
+// The one-wave form: a wave per tile does everything, with the steps in a ring
+// of 6 slices in registers.  Its chain is longer (20 instructions a step with
+// one channel), but a tile issues half the instructions that a front wave and
+// its producers do, which counts where a pass has more tiles than compute
+// units can serve at once (see kRowWaveTiles).
+constexpr int kRowWaveMaxK = 24;
+template <int CT, bool LAMB1, bool FAST, bool INIT>
+__device__ __forceinline__ void row_wave_run(const SweepDesc &Dd, const RowTile &T, int K, unsigned tag_base,
+                                             gu64 *__restrict__ halo, int *__restrict__ status, int spin_limit,
+                                             unsigned *xhist_wg) {
+  constexpr int P = kRowHaloStep;
+  struct Step {
+    float I[CT], d;
+  } S[P];
+  const __amdgpu_buffer_rsrc_t rd =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(INIT ? Dd.init_src : Dd.d), 0, T.range, 0x00020000);
+  auto load = [&](Step &q, unsigned o) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const __amdgpu_buffer_rsrc_t ri =
+          __builtin_amdgcn_make_buffer_rsrc((void *)(Dd.img + c * Dd.cs), 0, T.range, 0x00020000);
+      q.I[c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ri, (int)o, 0, 0));
+    }
+    q.d = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rd, (int)o, 0, 0));
+  };
+  const bool init_inv = Dd.init_mode == 2;
+  auto init_of = [&](float m) {
+    const float t = 1.0f - m;
+    return INIT ? Dd.init_v * (init_inv ? t : m) : m;
+  };
+  // stores: the sweep's own layout or the other one, at out0 + a * outA
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(Dd.dxo ? Dd.dxo : Dd.d), 0, T.range, 0x00020000);
+  const unsigned outA = Dd.dxo ? (unsigned)Dd.sXa * 4u : T.stride4;
+  const unsigned out0 = Dd.dxo ? (unsigned)T.e * (unsigned)Dd.sXe * 4u : T.lofs;
+  const float e1s = Dd.e1[3], e1c = Dd.e1[4], e1n = Dd.e1[5], lg = Dd.lg;
+
+  const int a0 = T.a_first - T.dir;  // the sweep's untouched first slice
+  load(S[P - 1], row_ofs(T, a0));
+  float F = T.lane_valid ? init_of(S[P - 1].d) : kInf;
+  if (T.lane_own && (Dd.dxo || INIT))
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F), rs, (int)(out0 + (unsigned)a0 * outA), 0, 0);
+  unsigned pf = row_ofs(T, T.a_first);
+#pragma unroll
+  for (int p = 0; p < P - 1; ++p, pf += T.dstride4) load(S[p], pf);
+
+  // Step s with its slice in S[slot] and the front's image in the slot before,
+  // which is then refilled with the slice of step s + P - 1.
+  auto step = [&](int slot, int s, bool prefetch) {
+    Step &Fr = S[(slot + P - 1) % P], &Sl = S[slot];
+    const float c3 = candidate<1, 0, CT, LAMB1>(F, Fr.I, Sl.I, e1s, lg);
+    const float c4 = candidate<1, 1, CT, LAMB1>(F, Fr.I, Sl.I, e1c, lg);
+    const float c5 = candidate<1, 2, CT, LAMB1>(F, Fr.I, Sl.I, e1n, lg);
+    float nd = init_of(Sl.d);
+    if constexpr (FAST) {
+      const float m = fminf(fminf(c3, c4), c5);
+      nd = (m < nd) ? m : nd;
+    } else {
+      nd = (c3 < nd) ? c3 : nd;
+      nd = (c4 < nd) ? c4 : nd;
+      nd = (c5 < nd) ? c5 : nd;
+    }
+    F = T.lane_valid ? nd : kInf;
+    // (padded steps of the last block and lanes of other tiles store nothing)
+    const unsigned o = out0 + (unsigned)(T.a_first + s * T.dir) * outA;
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F), rs, (int)(T.lane_own && s < T.nsteps ? o : 0xFFFFFFFFu),
+                                          0, 0);
+    if (prefetch) {
+      load(Fr, pf);
+      pf += T.dstride4;
+    }
+  };
+  const int nTE = Dd.nTE, TE = Dd.TE, te = T.te;
+  const bool pub = T.lane_own && ((te > 0 && T.e - T.e_own0 < K) || (te < nTE - 1 && T.e_own1 - 1 - T.e < K));
+  const bool need = T.lane_valid && !T.lane_own && max(T.e_own0 - T.e, T.e - (T.e_own1 - 1)) <= K;
+  const int ote = T.lane_valid ? T.e / TE : te;
+  gu64 *pub_at = halo + (long long)te * 2 * TE + (T.lane_own ? T.e - T.e_own0 : 0);
+  const gu64 *src_at = halo + (long long)ote * 2 * TE + (T.lane_valid ? T.e - ote * TE : 0);
+  bool tripped = false;
+  for (int b = 0;; ++b) {
+    int s = b * K;
+    for (int g = 1; g < K / P; ++g, s += P) {
+#pragma unroll
+      for (int p = 0; p < P; ++p) step(p, s + p, true);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) step(p, s + p, p < P - 1);  // (the last prefetch follows the poll below)
+    if (b + 1 >= T.nblocks) break;
+    const unsigned long long t_in = xhist_wg ? wall_clock64() : 0ull;
+    const unsigned tag = tag_base + (unsigned)(b + 1);
+    const int hslot = ((b + 1) & 1) * TE;
+    if (pub) __hip_atomic_store(pub_at + hslot, pack(F, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_sleep(kRowPollDelay);
+    unsigned long long x = (unsigned long long)tag << 32;
+    if (need) x = __hip_atomic_load(src_at + hslot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    load(S[P - 2], pf);
+    pf += T.dstride4;
+    // (bounded as in row_sweep_kernel)
+    int spins = tripped ? spin_limit : 0;
+    while ((unsigned)(x >> 32) != tag) {
+      if (++spins > spin_limit) {
+        __hip_atomic_store(status, FG_EWATCHDOG, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        tripped = true;
+        break;
+      }
+      x = __hip_atomic_load(src_at + hslot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (need) F = __uint_as_float((unsigned)x);
+    if (xhist_wg && T.lane == 0) {
+      const unsigned long long dt = wall_clock64() - t_in;
+      atomicAdd(&xhist_wg[dt ? min(64 - __clzll(dt), kXHistBuckets - 1) : 0], 1u);
+    }
+  }
+}
+
+template <bool LAMB1, bool FAST>
+__global__ __launch_bounds__(64) void row_wave_kernel(
+    const SweepDesc *__restrict__ descs, int ndesc, SweepDesc one, int K, unsigned tag_base,
+    unsigned long long *__restrict__ halo_base, int *__restrict__ status, int spin_limit,
+    unsigned *__restrict__ xhist) {
+  __shared__ unsigned xhist_wg[kXHistBuckets];
+  const int tile = xcd_remap(blockIdx.x, gridDim.x);
+  if (xhist) {
+    if (threadIdx.x < kXHistBuckets) xhist_wg[threadIdx.x] = 0u;
+    __syncthreads();
+  }
+  SweepDesc Dd;
+  if (descs) {
+    int lo = 0, hi = ndesc - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (descs[mid].tile0 <= tile) lo = mid; else hi = mid - 1;
+    }
+    Dd = descs[lo];
+  } else {
+    Dd = one;
+  }
+  // (the prefetch runs K + P - 2 slices past the end at most: see row_ofs)
+  static_assert(kRowWaveMaxK + kRowHaloStep - 2 <= 32, "prefetches past the end stay out of range");
+  if (K <= 0 || K % kRowHaloStep != 0 || K > kRowWaveMaxK || Dd.nB != 1 || Dd.C < 1 || Dd.C > 4) {
+    if (threadIdx.x == 0) __hip_atomic_store(status, FG_EINVAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  const RowTile T = row_tile(Dd, tile - Dd.tile0, K);
+  if (T.nsteps <= 0) return;
+  gu64 *const halo = (gu64 *)halo_base + Dd.halo0;
+  unsigned *const xh = xhist ? xhist_wg : nullptr;
+  auto run = [&](auto ct) {
+    constexpr int CT = decltype(ct)::value;
+    if (Dd.init_mode) row_wave_run<CT, LAMB1, FAST, true>(Dd, T, K, tag_base, halo, status, spin_limit, xh);
+    else row_wave_run<CT, LAMB1, FAST, false>(Dd, T, K, tag_base, halo, status, spin_limit, xh);
+  };
+  switch (Dd.C) {
+    case 1: run(std::integral_constant<int, 1>{}); break;
+    case 2: run(std::integral_constant<int, 2>{}); break;
+    case 3: run(std::integral_constant<int, 3>{}); break;
+    default: run(std::integral_constant<int, 4>{}); break;
   }
   if (xhist) {
     __syncthreads();
@@ -2118,7 +2288,12 @@ const void *pick_row_variant(bool lamb1, bool fast) {
               : reinterpret_cast<const void *>(&row_sweep_kernel<K, false, false>);
 }
 
-const void *pick_row_kernel(int K, bool lamb1, bool fast) {
+const void *pick_row_kernel(int K, bool lamb1, bool fast, bool wave) {
+  if (wave) {
+    if (lamb1) return reinterpret_cast<const void *>(&row_wave_kernel<true, true>);
+    return fast ? reinterpret_cast<const void *>(&row_wave_kernel<false, true>)
+                : reinterpret_cast<const void *>(&row_wave_kernel<false, false>);
+  }
   switch (K) {
     case 6: return pick_row_variant<6>(lamb1, fast);
     case 12: return pick_row_variant<12>(lamb1, fast);
@@ -2464,15 +2639,25 @@ struct SweepJob {
 
 // What the sweeps of one launch share.  Row sweeps (row()) of any channel
 // count, output form and initialisation share a kernel: C, xs and in are 0.
+// Row launches of more tiles than this a compute unit run the one-wave form.
+// Front and producers / one wave, ms a call: 32 RGB 1024^2 GSF iter 4 (2560
+// tiles) 31.4 / 20.6, 24 RGB 2000 x 1500 signed (1872) 8.6 / 7.9, 48 of 1500 x
+// 2000 (1872) 7.4 / 7.0, 64 of 512^2 (832) 1.31 / 1.26; below the line a
+// 1252 x 1292 GSF (324 tiles at K = 24) 1.3 / 2.1.  The one-wave form's tiles
+// leave the layout change to transposes: storing the other layout themselves
+// (runs of K elements a lane) they took 28.8 instead of 20.6 ms on the first.
+constexpr int kRowWaveTiles = 3;
+
 struct SweepGroup {
   int NW, R, P, K, C;
   bool l1, fa;
   int xs;
   bool in, cm;
   bool row() const { return NW == 1; }
-  int threads() const { return row() ? kRowThreads : (NW + (cm ? kCommWaves : 0)) * 64; }
+  bool wave = false;  // rows: the one-wave form
+  int threads() const { return row() ? (wave ? 64 : kRowThreads) : (NW + (cm ? kCommWaves : 0)) * 64; }
   const void *kernel() const {
-    return row() ? pick_row_kernel(K, l1, fa) : pick_kernel(NW, R, P, C, l1, fa, xs, in, cm);
+    return row() ? pick_row_kernel(K, l1, fa, wave) : pick_kernel(NW, R, P, C, l1, fa, xs, in, cm);
   }
   bool operator==(const SweepGroup &o) const {
     return NW == o.NW && R == o.R && P == o.P && K == o.K && C == o.C && l1 == o.l1 && fa == o.fa && xs == o.xs &&
@@ -2807,6 +2992,21 @@ struct Runner {
     return (t16 > 0 && t16 <= dev.cus) ? kSmallPlaneShape : g_shape;
   }
 
+  // Whether the launch of row transform i has tiles for the one-wave form
+  // (kRowWaveTiles; record_group decides by the same count).
+  bool many_rows(const std::vector<Xform *> &active, int pass, const std::vector<int> &ks, size_t i) {
+    if (ks[i] > kRowWaveMaxK) return false;
+    long long all = 0;
+    for (size_t j = 0; j < active.size(); ++j) {
+      const Xform *x = active[j];
+      int nA, nB, nE;
+      pass_plane(*x, pass, nA, nB, nE);
+      if (nB == 1 && nA > 1 && ks[j] == ks[i] && x->lamb1 == active[i]->lamb1 && x->fast == active[i]->fast)
+        all += plan_fixed(nB, nE, ks[j], x->C).nTE;
+    }
+    return all > (long long)kRowWaveTiles * dev.cus;
+  }
+
   // Record one pass (forward then backward) for the active transforms.
   int sweep_pass(std::vector<Xform *> &active, int pass) {
     ShapeScope shape_scope(pass_shape(active, pass));
@@ -2835,12 +3035,12 @@ struct Runner {
         int xs = 0;
         if (pass == 1 && dir < 0 && x->xst) {
           // (the pass may run on a shape without a B-contiguous kernel)
-          if (x->is2d) xs = 2;
+          if (x->is2d && !many_rows(active, pass, ks, i)) xs = 2;
           else if (p.NW > 1 && pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 1, in, p.comm)) xs = 1;
           else x->xst = false;
         }
         if (pass == 2 && dir < 0 && x->xsa) {
-          if (x->is2d ||
+          if ((x->is2d && !many_rows(active, pass, ks, i)) ||
               (p.nTB > 1 && p.K <= kXsaMaxK && pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 2, in, p.comm)))
             xs = 2;
           else
@@ -2869,6 +3069,20 @@ struct Runner {
     int rc = coresident_groups(kern, g.threads(), dev, cap);
     if (rc) return rc;
     if (max_groups > 0) cap = std::min<long long>(cap, max_groups);
+    if (g.row() && !g.wave && g.K <= kRowWaveMaxK) {
+      long long all = 0;
+      for (auto &j : jobs) {
+        int nA, nB, nE;
+        pass_plane(*j.x, j.pass, nA, nB, nE);
+        const Plan p = plan_fixed(nB, nE, j.K, j.x->C);
+        all += (long long)p.nTB * p.nTE;
+      }
+      if (all > (long long)kRowWaveTiles * dev.cus) {
+        SweepGroup one = g;
+        one.wave = true;
+        return record_group(jobs, dir, one);
+      }
+    }
     // A launch lasts as long as its longest sweep: pack planes of similar
     // step counts together (longest first).
     std::stable_sort(jobs.begin(), jobs.end(), [](const SweepJob &u, const SweepJob &v) {
@@ -3034,7 +3248,8 @@ struct Runner {
     pass_plane(x, pass, nA, nB, nE);
     const Plan p = plan_fixed(nB, nE, K > 0 ? K : 1, x.C);
     if (!p.ok) return FG_OK;
-    const SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm};
+    SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm};
+    g.wave = g.row() && (long long)p.nTE > (long long)kRowWaveTiles * dev.cus && g.K <= kRowWaveMaxK;
     const void *kern = g.kernel();
     if (!kern) return FG_OK;
     long long cap = 0;

@@ -110,3 +110,29 @@ def test_small_images(device, C, H, W, lamb):
     got = FG.geodesic_batch(insts)
     assert equal(got[0].cpu().numpy(), oracle.py_geodesic2d(big, bm, 1e10, lamb, 2))
     assert all(equal(g.cpu().numpy(), want) for g in got[1:])
+
+
+@pytest.mark.parametrize("lamb", [1.0, 0.5, 1.5])
+@pytest.mark.parametrize("K", [0, 6, 12, 18, 24])
+def test_many_tiles(device, lamb, K):
+    """Launches of more tiles than the front-and-producers form is used for:
+    1-4 channels, initialising and later sweeps, lengths around one and two
+    blocks, both output layouts, NaN and infinities."""
+    rng = np.random.default_rng(23 + K)
+    insts, wants = [], []
+    for k in range(44):
+        C, n = 1 + k % 4, (2, 5, 6, 7, 13, 25, 31, 49)[k % 8]
+        H, W = (n, 1200 + k) if k % 2 else (1200 + k, n)
+        img, m = make(rng, C, H, W, special=k % 5 == 0)
+        with np.errstate(all="ignore"):
+            wants.append(oracle.py_geodesic2d(img, m, 1e10, lamb, 2))
+        insts.append(FG.Instance(torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda(), 1e10, lamb, iter=2))
+    insts, wants = insts + insts, wants + wants  # (rows of one half, columns of the other: > 900 tiles each)
+    old = FG.get_tuning()
+    FG.set_tuning(halo=K)
+    try:
+        print(f"many tiles lamb={lamb} K={K}", flush=True)
+        for got, want in zip(FG.geodesic_batch(insts), wants):
+            assert equal(got.cpu().numpy(), want)
+    finally:
+        FG.set_tuning(**old)
