@@ -1428,25 +1428,25 @@ __device__ __forceinline__ void row_wave_run(const SweepDesc &Dd, const RowTile 
     const float t = 1.0f - m;
     return INIT ? Dd.init_v * (init_inv ? t : m) : m;
   };
-  // stores: the sweep's own layout or the other one, at out0 + a * outA
-  const __amdgpu_buffer_rsrc_t rs =
-      __builtin_amdgcn_make_buffer_rsrc((void *)(Dd.dxo ? Dd.dxo : Dd.d), 0, T.range, 0x00020000);
-  const unsigned outA = Dd.dxo ? (unsigned)Dd.sXa * 4u : T.stride4;
-  const unsigned out0 = Dd.dxo ? (unsigned)T.e * (unsigned)Dd.sXe * 4u : T.lofs;
+  // stores: the offsets of slices past either end and, based at 2^31, of lanes
+  // of other tiles are out of range (see row_ofs)
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)Dd.d, 0, T.range, 0x00020000);
+  const unsigned out0 = T.lane_own ? T.lofs : 0x80000000u;
+  unsigned st = (unsigned)T.a_first * T.stride4;
   const float e1s = Dd.e1[3], e1c = Dd.e1[4], e1n = Dd.e1[5], lg = Dd.lg;
 
   const int a0 = T.a_first - T.dir;  // the sweep's untouched first slice
   load(S[P - 1], row_ofs(T, a0));
   float F = T.lane_valid ? init_of(S[P - 1].d) : kInf;
-  if (T.lane_own && (Dd.dxo || INIT))
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F), rs, (int)(out0 + (unsigned)a0 * outA), 0, 0);
+  if (INIT)
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F), rs, (int)(out0 + (unsigned)a0 * T.stride4), 0, 0);
   unsigned pf = row_ofs(T, T.a_first);
 #pragma unroll
   for (int p = 0; p < P - 1; ++p, pf += T.dstride4) load(S[p], pf);
 
-  // Step s with its slice in S[slot] and the front's image in the slot before,
-  // which is then refilled with the slice of step s + P - 1.
-  auto step = [&](int slot, int s, bool prefetch) {
+  // The next step, with its slice in S[slot] and the front's image in the slot
+  // before, which is then refilled with the slice P - 1 steps on.
+  auto step = [&](int slot, bool prefetch) {
     Step &Fr = S[(slot + P - 1) % P], &Sl = S[slot];
     const float c3 = candidate<1, 0, CT, LAMB1>(F, Fr.I, Sl.I, e1s, lg);
     const float c4 = candidate<1, 1, CT, LAMB1>(F, Fr.I, Sl.I, e1c, lg);
@@ -1461,10 +1461,8 @@ __device__ __forceinline__ void row_wave_run(const SweepDesc &Dd, const RowTile 
       nd = (c5 < nd) ? c5 : nd;
     }
     F = T.lane_valid ? nd : kInf;
-    // (padded steps of the last block and lanes of other tiles store nothing)
-    const unsigned o = out0 + (unsigned)(T.a_first + s * T.dir) * outA;
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F), rs, (int)(T.lane_own && s < T.nsteps ? o : 0xFFFFFFFFu),
-                                          0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(F), rs, (int)(out0 + st), 0, 0);
+    st += T.dstride4;
     if (prefetch) {
       load(Fr, pf);
       pf += T.dstride4;
@@ -1478,13 +1476,12 @@ __device__ __forceinline__ void row_wave_run(const SweepDesc &Dd, const RowTile 
   const gu64 *src_at = halo + (long long)ote * 2 * TE + (T.lane_valid ? T.e - ote * TE : 0);
   bool tripped = false;
   for (int b = 0;; ++b) {
-    int s = b * K;
-    for (int g = 1; g < K / P; ++g, s += P) {
+    for (int g = 1; g < K / P; ++g) {
 #pragma unroll
-      for (int p = 0; p < P; ++p) step(p, s + p, true);
+      for (int p = 0; p < P; ++p) step(p, true);
     }
 #pragma unroll
-    for (int p = 0; p < P; ++p) step(p, s + p, p < P - 1);  // (the last prefetch follows the poll below)
+    for (int p = 0; p < P; ++p) step(p, p < P - 1);  // (the last prefetch follows the poll below)
     if (b + 1 >= T.nblocks) break;
     const unsigned long long t_in = xhist_wg ? wall_clock64() : 0ull;
     const unsigned tag = tag_base + (unsigned)(b + 1);
@@ -1537,7 +1534,7 @@ __global__ __launch_bounds__(64) void row_wave_kernel(
   }
   // (the prefetch runs K + P - 2 slices past the end at most: see row_ofs)
   static_assert(kRowWaveMaxK + kRowHaloStep - 2 <= 32, "prefetches past the end stay out of range");
-  if (K <= 0 || K % kRowHaloStep != 0 || K > kRowWaveMaxK || Dd.nB != 1 || Dd.C < 1 || Dd.C > 4) {
+  if (K <= 0 || K % kRowHaloStep != 0 || K > kRowWaveMaxK || Dd.nB != 1 || Dd.dxo || Dd.C < 1 || Dd.C > 4) {
     if (threadIdx.x == 0) __hip_atomic_store(status, FG_EINVAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return;
   }
@@ -2641,11 +2638,10 @@ struct SweepJob {
 // count, output form and initialisation share a kernel: C, xs and in are 0.
 // Row launches of more tiles than this a compute unit run the one-wave form.
 // Front and producers / one wave, ms a call: 32 RGB 1024^2 GSF iter 4 (2560
-// tiles) 31.4 / 20.6, 24 RGB 2000 x 1500 signed (1872) 8.6 / 7.9, 48 of 1500 x
-// 2000 (1872) 7.4 / 7.0, 64 of 512^2 (832) 1.31 / 1.26; below the line a
+// tiles) 31.4 / 20.3, 64 of 512^2 (832) 1.31 / 1.20; below the line a
 // 1252 x 1292 GSF (324 tiles at K = 24) 1.3 / 2.1.  The one-wave form's tiles
 // leave the layout change to transposes: storing the other layout themselves
-// (runs of K elements a lane) they took 28.8 instead of 20.6 ms on the first.
+// (runs of K elements a lane) they took 28.8 ms on the first.
 constexpr int kRowWaveTiles = 3;
 
 struct SweepGroup {
@@ -3071,13 +3067,15 @@ struct Runner {
     if (max_groups > 0) cap = std::min<long long>(cap, max_groups);
     if (g.row() && !g.wave && g.K <= kRowWaveMaxK) {
       long long all = 0;
+      bool xs = false;  // (it writes the sweep's own layout only)
       for (auto &j : jobs) {
+        xs = xs || j.xs != 0;
         int nA, nB, nE;
         pass_plane(*j.x, j.pass, nA, nB, nE);
         const Plan p = plan_fixed(nB, nE, j.K, j.x->C);
         all += (long long)p.nTB * p.nTE;
       }
-      if (all > (long long)kRowWaveTiles * dev.cus) {
+      if (!xs && all > (long long)kRowWaveTiles * dev.cus) {
         SweepGroup one = g;
         one.wave = true;
         return record_group(jobs, dir, one);
