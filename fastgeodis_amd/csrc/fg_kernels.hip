@@ -2185,21 +2185,31 @@ Plan plan_fixed(int nB, int nE, int Kreq, int C, int shape = -1) {
   return p;
 }
 
+// Tiles that a plan counts on: one 3D tile a compute unit, of rows as many
+// workgroups as a unit serves at halo depth K, and never more than a workgroup
+// cap (max_groups) allows in one launch.
+struct TileBudget {
+  int cus, max_groups;
+  long long of(int nB, int K) const {
+    const long long n = nB == 1 ? (long long)cus * row_groups_per_cu(K) : cus;
+    return max_groups > 0 ? std::min<long long>(n, max_groups) : n;
+  }
+};
+
 // Plan of one sweep plane.  Kreq > 0: that halo depth, rounded up to a
 // multiple of the slab ring (a row whose tiles would not all be resident at
 // that depth takes the deepest at which they are, in a 3D volume one whose
 // entries fit the exchange buffer of the requested depth).  Kreq == 0 (automatic):
-// the deepest halo (fewest exchanges) whose tiles still fit one per compute
-// unit (rows: row_groups_per_cu), as every tile waits for its neighbours at
-// each exchange; if even the shallowest halo needs more tiles, that one.
-Plan plan_plane(int nB, int nE, int Kreq, int C, int tile_budget, bool is2d) {
-  auto budget = [&](int K) { return nB == 1 ? tile_budget * row_groups_per_cu(K) : tile_budget; };
+// the deepest halo (fewest exchanges) whose tiles still fit the budget, as
+// every tile waits for its neighbours at each exchange; if even the shallowest
+// halo, which has the fewest tiles, needs more, that one.
+Plan plan_plane(int nB, int nE, int Kreq, int C, const TileBudget &budget, bool is2d) {
   if (Kreq > 0) {
     const Plan p = plan_fixed(nB, nE, Kreq, C);
-    if (nB > 1 || p.nTE <= 2 * tile_budget) return p;
+    if (nB > 1 || p.nTE <= 2 * budget.cus) return p;
     for (int K = p.K - p.P; K > 0; K -= p.P) {
       const Plan q = plan_fixed(nB, nE, K, C);
-      if ((q.nTE <= 2 * tile_budget || K == p.P) && (is2d || q.nTE * q.TE <= p.nTE * p.TE)) return q;
+      if ((q.nTE <= 2 * budget.cus || K == p.P) && (is2d || q.nTE * q.TE <= p.nTE * p.TE)) return q;
     }
     return p;
   }
@@ -2208,7 +2218,7 @@ Plan plan_plane(int nB, int nE, int Kreq, int C, int tile_budget, bool is2d) {
   for (int K = first.P; K <= kMaxK; K += first.P) {
     const Plan q = plan_fixed(nB, nE, K, C);
     if (!q.ok) break;
-    if ((long long)q.nTB * q.nTE > budget(K)) continue;
+    if ((long long)q.nTB * q.nTE > budget.of(nB, K)) continue;
     best = q;
   }
   return best;
@@ -2672,6 +2682,8 @@ struct Runner {
 
   bool no_graph = false;  // replay the launches directly (sequences that do not repeat)
 
+  TileBudget budget() const { return {dev.cus, max_groups}; }
+
   void fill_desc(const Xform &x, int pass, int dir, SweepDesc &s, int xs = 0) {
     std::memset(&s, 0, sizeof s);
     if (x.init_mode && x.it == 0 && pass == first_pass(x) && dir > 0) {
@@ -2723,7 +2735,7 @@ struct Runner {
     int nA, nB, nE;
     pass_plane(x, 1, nA, nB, nE);
     if (nA <= 1 || nB <= 1) return false;
-    const Plan p = plan_plane(nB, nE, K, x.C, dev.cus, x.is2d);
+    const Plan p = plan_plane(nB, nE, K, x.C, budget(), x.is2d);
     if (!p.ok || !pick_kernel(p.NW, p.R, p.P, x.C, x.lamb1, x.fast, 1, false, p.comm)) return false;
     if ((long long)x.D * x.H * x.W * 4 >= 0xFFFFFFF0ll) return false;
     return slice_offsets_fit(x, 1);
@@ -2906,7 +2918,7 @@ struct Runner {
     int nA, nB, nE;
     pass_plane(x, pass, nA, nB, nE);
     if (nA <= 1 || engine == 0 || x.C > 4) return false;
-    return plan_plane(nB, nE, K, x.C, dev.cus, x.is2d).ok && slice_offsets_fit(x, pass);
+    return plan_plane(nB, nE, K, x.C, budget(), x.is2d).ok && slice_offsets_fit(x, pass);
   }
 
   // Halo depth of each transform's plane in this pass.  Requested depths
@@ -2926,7 +2938,7 @@ struct Runner {
       int nA, nB, nE;
       pass_plane(*active[i], pass, nA, nB, nE);
       if (!tiled_eligible(*active[i], pass)) continue;
-      ks[i] = plan_plane(nB, nE, K, active[i]->C, dev.cus, active[i]->is2d).K;
+      ks[i] = plan_plane(nB, nE, K, active[i]->C, budget(), active[i]->is2d).K;
       if (K == 0) (nB > 1 ? planes : rows).push_back((int)i);
     }
     if (rows.size() > 1) share_halo(active, pass, rows, ks);
@@ -2949,19 +2961,19 @@ struct Runner {
     for (int P : rings) {
       int best = P;
       for (int k = P; k <= kMaxK; k += P) {
-        long long tiles = 0, budget = dev.cus;
+        long long tiles = 0, fits = 0;
         bool ok = true;
         for (int i : idx) {
           if (ring(i) != P) continue;
           int nA, nB, nE;
           pass_plane(*active[i], pass, nA, nB, nE);
-          if (nB == 1) budget = (long long)dev.cus * row_groups_per_cu(k);
+          fits = budget().of(nB, k);
           const Plan q = plan_fixed(nB, nE, k, active[i]->C);
           if (!q.ok) { ok = false; break; }
           tiles += (long long)q.nTB * q.nTE;
         }
         if (!ok) break;
-        if (tiles <= budget) best = k;
+        if (tiles <= fits) best = k;
       }
       for (int i : idx)
         if (ring(i) == P) ks[i] = best;
@@ -2985,7 +2997,7 @@ struct Runner {
       if (!a.ok || !b.ok || a.nTB == 1) return g_shape;
       t16 += (long long)b.nTB * b.nTE;
     }
-    return (t16 > 0 && t16 <= dev.cus) ? kSmallPlaneShape : g_shape;
+    return (t16 > 0 && t16 <= budget().of(2, 5)) ? kSmallPlaneShape : g_shape;
   }
 
   // Whether the launch of row transform i has tiles for the one-wave form
@@ -3236,8 +3248,10 @@ struct Runner {
   }
 
   // Whether the first sweep of x runs on the tiled engine whatever halo depth
-  // its pass is planned with (the plane fits the device's co-resident
-  // workgroups even at the shallowest halo, which has the most tiles).
+  // and shape its pass is planned with: the plane's tiles at the shallowest
+  // halo, which has the fewest, are co-resident (and within a workgroup cap).
+  // Deeper halos and 16-row windows are planned only where their tiles fit
+  // the budget, which is within both.
   int first_sweep_tiled(const Xform &x, bool &tiled) {
     tiled = false;
     const int pass = first_pass(x);
