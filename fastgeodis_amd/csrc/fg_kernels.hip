@@ -2644,8 +2644,6 @@ struct SweepJob {
   int xs;  // output form (SweepDesc::dxo)
 };
 
-// What the sweeps of one launch share.  Row sweeps (row()) of any channel
-// count, output form and initialisation share a kernel: C, xs and in are 0.
 // Row launches of more tiles than this a compute unit run the one-wave form.
 // Front and producers / one wave, ms a call: 32 RGB 1024^2 GSF iter 4 (2560
 // tiles) 31.4 / 20.3, 64 of 512^2 (832) 1.31 / 1.20; below the line a
@@ -2654,20 +2652,22 @@ struct SweepJob {
 // (runs of K elements a lane) they took 28.8 ms on the first.
 constexpr int kRowWaveTiles = 3;
 
+// What the sweeps of one launch share.  Row sweeps (row()) of any channel
+// count, output form and initialisation share a kernel: C, xs and in are 0.
 struct SweepGroup {
   int NW, R, P, K, C;
   bool l1, fa;
   int xs;
   bool in, cm;
+  bool wave;  // rows: the one-wave form
   bool row() const { return NW == 1; }
-  bool wave = false;  // rows: the one-wave form
   int threads() const { return row() ? (wave ? 64 : kRowThreads) : (NW + (cm ? kCommWaves : 0)) * 64; }
   const void *kernel() const {
     return row() ? pick_row_kernel(K, l1, fa, wave) : pick_kernel(NW, R, P, C, l1, fa, xs, in, cm);
   }
   bool operator==(const SweepGroup &o) const {
     return NW == o.NW && R == o.R && P == o.P && K == o.K && C == o.C && l1 == o.l1 && fa == o.fa && xs == o.xs &&
-           in == o.in && cm == o.cm;
+           in == o.in && cm == o.cm && wave == o.wave;
   }
 };
 
@@ -3000,25 +3000,36 @@ struct Runner {
     return (t16 > 0 && t16 <= budget().of(2, 5)) ? kSmallPlaneShape : g_shape;
   }
 
-  // Whether the launch of row transform i has tiles for the one-wave form
-  // (kRowWaveTiles; record_group decides by the same count).
-  bool many_rows(const std::vector<Xform *> &active, int pass, const std::vector<int> &ks, size_t i) {
-    if (ks[i] > kRowWaveMaxK) return false;
-    long long all = 0;
-    for (size_t j = 0; j < active.size(); ++j) {
-      const Xform *x = active[j];
+  // Whether a row launch of that many tiles at halo depth K runs the one-wave
+  // form.
+  bool row_wave(long long tiles, int K) const {
+    return K <= kRowWaveMaxK && tiles > (long long)kRowWaveTiles * dev.cus;
+  }
+
+  // Which of a pass's transforms run on it: the rows that share a launch (same
+  // depth, lamb class and fold) are counted together, once for the pass (a
+  // count per transform made the recording of a batch quadratic: 1024 images of
+  // 150 x 170 12.3 ms a call instead of 6.9).
+  std::vector<char> row_waves(const std::vector<Xform *> &active, int pass, const std::vector<int> &ks) const {
+    long long tiles[kMaxK + 1][2][2] = {};
+    std::vector<char> is_row(active.size(), 0), wave(active.size(), 0);
+    for (size_t i = 0; i < active.size(); ++i) {
+      const Xform *x = active[i];
       int nA, nB, nE;
       pass_plane(*x, pass, nA, nB, nE);
-      if (nB == 1 && nA > 1 && ks[j] == ks[i] && x->lamb1 == active[i]->lamb1 && x->fast == active[i]->fast)
-        all += plan_fixed(nB, nE, ks[j], x->C).nTE;
+      is_row[i] = nB == 1 && nA > 1 && ks[i] > 0;
+      if (is_row[i]) tiles[ks[i]][x->lamb1][x->fast] += plan_fixed(nB, nE, ks[i], x->C).nTE;
     }
-    return all > (long long)kRowWaveTiles * dev.cus;
+    for (size_t i = 0; i < active.size(); ++i)
+      wave[i] = is_row[i] && row_wave(tiles[ks[i]][active[i]->lamb1][active[i]->fast], ks[i]);
+    return wave;
   }
 
   // Record one pass (forward then backward) for the active transforms.
   int sweep_pass(std::vector<Xform *> &active, int pass) {
     ShapeScope shape_scope(pass_shape(active, pass));
     const std::vector<int> ks = pass_halos(active, pass);
+    const std::vector<char> wave = row_waves(active, pass, ks);
     for (int dir : {+1, -1}) {
       std::vector<std::pair<SweepGroup, std::vector<SweepJob>>> groups;
       for (size_t i = 0; i < active.size(); ++i) {
@@ -3036,19 +3047,20 @@ struct Runner {
         }
         const Plan p = plan_fixed(nB, nE, ks[i], x->C);
         // Backward sweeps that write the next layout themselves: 2D row tiles
-        // store every block from LDS in either layout; 3D tiles stage the own
+        // store every block from LDS in either layout (the one-wave form only
+        // its own); 3D tiles stage the own
         // rows of a tile of several along B, and the slices of one block
         // beyond a run.  Otherwise the distance moves between layouts through
         // a transpose.
         int xs = 0;
         if (pass == 1 && dir < 0 && x->xst) {
           // (the pass may run on a shape without a B-contiguous kernel)
-          if (x->is2d && !many_rows(active, pass, ks, i)) xs = 2;
+          if (x->is2d && !wave[i]) xs = 2;
           else if (p.NW > 1 && pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 1, in, p.comm)) xs = 1;
           else x->xst = false;
         }
         if (pass == 2 && dir < 0 && x->xsa) {
-          if ((x->is2d && !many_rows(active, pass, ks, i)) ||
+          if ((x->is2d && !wave[i]) ||
               (p.nTB > 1 && p.K <= kXsaMaxK && pick_kernel(p.NW, p.R, p.P, x->C, x->lamb1, x->fast, 2, in, p.comm)))
             xs = 2;
           else
@@ -3056,7 +3068,7 @@ struct Runner {
         }
         const bool row = p.NW == 1;
         const SweepGroup key{p.NW, p.R, p.P, p.K, row ? 0 : x->C, x->lamb1, x->fast, row ? 0 : xs, row ? false : in,
-                             p.comm};
+                             p.comm, wave[i] != 0};
         auto g = std::find_if(groups.begin(), groups.end(), [&](const auto &q) { return q.first == key; });
         if (g == groups.end()) g = groups.insert(groups.end(), {key, {}});
         g->second.push_back({x, pass, p.K, xs});
@@ -3077,22 +3089,6 @@ struct Runner {
     int rc = coresident_groups(kern, g.threads(), dev, cap);
     if (rc) return rc;
     if (max_groups > 0) cap = std::min<long long>(cap, max_groups);
-    if (g.row() && !g.wave && g.K <= kRowWaveMaxK) {
-      long long all = 0;
-      bool xs = false;  // (it writes the sweep's own layout only)
-      for (auto &j : jobs) {
-        xs = xs || j.xs != 0;
-        int nA, nB, nE;
-        pass_plane(*j.x, j.pass, nA, nB, nE);
-        const Plan p = plan_fixed(nB, nE, j.K, j.x->C);
-        all += (long long)p.nTB * p.nTE;
-      }
-      if (!xs && all > (long long)kRowWaveTiles * dev.cus) {
-        SweepGroup one = g;
-        one.wave = true;
-        return record_group(jobs, dir, one);
-      }
-    }
     // A launch lasts as long as its longest sweep: pack planes of similar
     // step counts together (longest first).
     std::stable_sort(jobs.begin(), jobs.end(), [](const SweepJob &u, const SweepJob &v) {
@@ -3260,8 +3256,7 @@ struct Runner {
     pass_plane(x, pass, nA, nB, nE);
     const Plan p = plan_fixed(nB, nE, K > 0 ? K : 1, x.C);
     if (!p.ok) return FG_OK;
-    SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm};
-    g.wave = g.row() && (long long)p.nTE > (long long)kRowWaveTiles * dev.cus && g.K <= kRowWaveMaxK;
+    const SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm, nB == 1 && row_wave(p.nTE, p.K)};
     const void *kern = g.kernel();
     if (!kern) return FG_OK;
     long long cap = 0;

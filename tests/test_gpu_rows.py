@@ -2,6 +2,8 @@
 wrong, bit for bit against the oracle: lines around one window (62-65 lanes),
 partial last tiles, sweeps of one step and around one and two blocks of every
 halo depth, NaN and infinite old distances, 1-4 channels in one launch."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -136,3 +138,25 @@ def test_many_tiles(device, lamb, K):
             assert equal(got.cpu().numpy(), want)
     finally:
         FG.set_tuning(**old)
+
+
+def test_recording_time_grows_with_the_batch(device):
+    """Host work per image does not grow with the batch: four times the images
+    take about four times as long (16 times where each image looks at all)."""
+    rng = np.random.default_rng(5)
+    img, m = make(rng, 1, 130, 20)
+    one = FG.Instance(torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda(), 1e10, 1.0, iter=1)
+
+    def took(n):
+        insts, best = [one] * n, float("inf")
+        for _ in range(4):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            FG.geodesic_batch(insts)
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        return best
+
+    few, many = took(1024), took(4096)
+    print(f"1024 images {few * 1e3:.1f} ms, 4096 images {many * 1e3:.1f} ms", flush=True)
+    assert many < 7 * few
