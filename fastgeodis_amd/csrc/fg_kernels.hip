@@ -1403,7 +1403,7 @@ __global__ __launch_bounds__(kRowThreads)
 // one channel), but a tile issues half the instructions that a front wave and
 // its producers do, which counts where a pass has more tiles than compute
 // units can serve at once (see kRowWaveTiles).
-constexpr int kRowWaveMaxK = 24;
+constexpr int kRowWaveMaxK = 30;
 template <int CT, bool LAMB1, bool FAST, bool INIT>
 __device__ __forceinline__ void row_wave_run(const SweepDesc &Dd, const RowTile &T, int K, unsigned tag_base,
                                              gu64 *__restrict__ halo, int *__restrict__ status, int spin_limit,
@@ -1532,8 +1532,11 @@ __global__ __launch_bounds__(64) void row_wave_kernel(
   } else {
     Dd = one;
   }
-  // (the prefetch runs K + P - 2 slices past the end at most: see row_ofs)
-  static_assert(kRowWaveMaxK + kRowHaloStep - 2 <= 32, "prefetches past the end stay out of range");
+  // A sweep's padded last block prefetches slices -(K + P - 3) .. nA + K + P - 4
+  // at most and stores to -(K - 1) .. nA + K - 2: with (nA + 32) slices in 2^31
+  // bytes, 33 slices to either side and stores based at 2^31 up to 32 of them
+  // stay between the array's range and 2^32.
+  static_assert(kRowWaveMaxK + kRowHaloStep - 3 <= 33 && kRowWaveMaxK <= 32, "slices past the ends stay out of range");
   if (K <= 0 || K % kRowHaloStep != 0 || K > kRowWaveMaxK || Dd.nB != 1 || Dd.dxo || Dd.C < 1 || Dd.C > 4) {
     if (threadIdx.x == 0) __hip_atomic_store(status, FG_EINVAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return;
@@ -2922,7 +2925,11 @@ struct Runner {
   }
 
   // Halo depth of each transform's plane in this pass.  Requested depths
-  // apply as they are.  Automatic: a lone plane takes the deepest halo whose
+  // apply as they are, but for rows that are too many for them (plan_plane;
+  // 2D rows at K = 30, 4 own lanes of 64, whose tiles together are not resident
+  // take K = 24: 48 images of 400 x 500 iter 2 at a requested 30 3.56 ms in
+  // launches of 512 tiles, 2.46 on the one-wave form, 0.98 at 24).
+  // Automatic: a lone plane takes the deepest halo whose
   // tiles fit one per CU (idle CUs cost nothing, and fewer exchanges shorten
   // the sweep).  Planes that share the pass (batches, the halves of a signed
   // or GSF call) are planned together: the deepest halo at which all their
@@ -2934,13 +2941,19 @@ struct Runner {
   std::vector<int> pass_halos(const std::vector<Xform *> &active, int pass) {
     std::vector<int> ks(active.size(), 0);
     std::vector<int> rows, planes;  // automatic 2D rows and 3D planes
+    long long deepest = 0;          // tiles of 2D rows at the deepest requested depth
     for (size_t i = 0; i < active.size(); ++i) {
       int nA, nB, nE;
       pass_plane(*active[i], pass, nA, nB, nE);
       if (!tiled_eligible(*active[i], pass)) continue;
-      ks[i] = plan_plane(nB, nE, K, active[i]->C, budget(), active[i]->is2d).K;
+      const Plan p = plan_plane(nB, nE, K, active[i]->C, budget(), active[i]->is2d);
+      ks[i] = p.K;
+      if (K > 0 && active[i]->is2d && p.K == kMaxK) deepest += p.nTE;
       if (K == 0) (nB > 1 ? planes : rows).push_back((int)i);
     }
+    if (deepest > 2 * dev.cus)
+      for (size_t i = 0; i < active.size(); ++i)
+        if (active[i]->is2d && ks[i] == kMaxK) ks[i] -= kRowHaloStep;
     if (rows.size() > 1) share_halo(active, pass, rows, ks);
     if (planes.size() > 1) share_halo(active, pass, planes, ks);
     return ks;
@@ -3000,36 +3013,58 @@ struct Runner {
     return (t16 > 0 && t16 <= budget().of(2, 5)) ? kSmallPlaneShape : g_shape;
   }
 
-  // Whether a row launch of that many tiles at halo depth K runs the one-wave
-  // form.
-  bool row_wave(long long tiles, int K) const {
-    return K <= kRowWaveMaxK && tiles > (long long)kRowWaveTiles * dev.cus;
+  // Whether a row launch runs the one-wave form: one of more tiles than
+  // kRowWaveTiles a compute unit, or with a plane (its widest) of more tiles
+  // than workgroups with a front and producers are resident at once (512 at
+  // K >= 24; a requested depth can ask for it).
+  int row_wave(long long tiles, long long widest, int K, bool lamb1, bool fast, bool &wave) const {
+    wave = tiles > (long long)kRowWaveTiles * dev.cus;
+    if (wave || widest <= dev.cus) return FG_OK;  // (at least one a compute unit is resident)
+    const void *kern = pick_row_kernel(K, lamb1, fast, false);
+    long long cap = 0;
+    if (!kern) return fail(FG_EINVAL, "no row kernel for this depth");
+    if (const int rc = coresident_groups(kern, kRowThreads, dev, cap)) return rc;
+    wave = widest > cap;
+    return FG_OK;
   }
 
   // Which of a pass's transforms run on it: the rows that share a launch (same
   // depth, lamb class and fold) are counted together, once for the pass (a
   // count per transform made the recording of a batch quadratic: 1024 images of
   // 150 x 170 12.3 ms a call instead of 6.9).
-  std::vector<char> row_waves(const std::vector<Xform *> &active, int pass, const std::vector<int> &ks) const {
-    long long tiles[kMaxK + 1][2][2] = {};
-    std::vector<char> is_row(active.size(), 0), wave(active.size(), 0);
+  int row_waves(const std::vector<Xform *> &active, int pass, const std::vector<int> &ks, std::vector<char> &wave) const {
+    struct Launch { long long tiles = 0, widest = 0; bool wave = false; };
+    Launch launch[kMaxK + 1][2][2];
+    wave.assign(active.size(), 0);
     for (size_t i = 0; i < active.size(); ++i) {
       const Xform *x = active[i];
       int nA, nB, nE;
       pass_plane(*x, pass, nA, nB, nE);
-      is_row[i] = nB == 1 && nA > 1 && ks[i] > 0;
-      if (is_row[i]) tiles[ks[i]][x->lamb1][x->fast] += plan_fixed(nB, nE, ks[i], x->C).nTE;
+      if (nB > 1 || nA <= 1 || ks[i] == 0) continue;
+      wave[i] = 1;  // a row
+      Launch &l = launch[ks[i]][x->lamb1][x->fast];
+      const int n = plan_fixed(nB, nE, ks[i], x->C).nTE;
+      l.tiles += n;
+      l.widest = std::max<long long>(l.widest, n);
     }
+    for (int k = 1; k <= kMaxK; ++k)
+      for (int lamb1 = 0; lamb1 < 2; ++lamb1)
+        for (int fast = 0; fast < 2; ++fast) {
+          Launch &l = launch[k][lamb1][fast];
+          if (l.tiles == 0) continue;
+          if (const int rc = row_wave(l.tiles, l.widest, k, lamb1, fast, l.wave)) return rc;
+        }
     for (size_t i = 0; i < active.size(); ++i)
-      wave[i] = is_row[i] && row_wave(tiles[ks[i]][active[i]->lamb1][active[i]->fast], ks[i]);
-    return wave;
+      wave[i] = wave[i] && launch[ks[i]][active[i]->lamb1][active[i]->fast].wave;
+    return FG_OK;
   }
 
   // Record one pass (forward then backward) for the active transforms.
   int sweep_pass(std::vector<Xform *> &active, int pass) {
     ShapeScope shape_scope(pass_shape(active, pass));
     const std::vector<int> ks = pass_halos(active, pass);
-    const std::vector<char> wave = row_waves(active, pass, ks);
+    std::vector<char> wave;
+    if (const int rc = row_waves(active, pass, ks, wave)) return rc;
     for (int dir : {+1, -1}) {
       std::vector<std::pair<SweepGroup, std::vector<SweepJob>>> groups;
       for (size_t i = 0; i < active.size(); ++i) {
@@ -3244,8 +3279,9 @@ struct Runner {
   }
 
   // Whether the first sweep of x runs on the tiled engine whatever halo depth
-  // and shape its pass is planned with: the plane's tiles at the shallowest
-  // halo, which has the fewest, are co-resident (and within a workgroup cap).
+  // and shape its pass is planned with: the plane's tiles at the requested
+  // depth's plan, or automatically at the shallowest halo, which has the
+  // fewest, are co-resident (and within a workgroup cap).
   // Deeper halos and 16-row windows are planned only where their tiles fit
   // the budget, which is within both.
   int first_sweep_tiled(const Xform &x, bool &tiled) {
@@ -3254,13 +3290,16 @@ struct Runner {
     if (x.iters <= 0 || !tiled_eligible(x, pass)) return FG_OK;
     int nA, nB, nE;
     pass_plane(x, pass, nA, nB, nE);
-    const Plan p = plan_fixed(nB, nE, K > 0 ? K : 1, x.C);
+    const Plan p = K > 0 ? plan_plane(nB, nE, K, x.C, budget(), x.is2d) : plan_fixed(nB, nE, 1, x.C);
     if (!p.ok) return FG_OK;
-    const SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm, nB == 1 && row_wave(p.nTE, p.K)};
+    bool wave = false;
+    int rc = FG_OK;
+    if (nB == 1 && (rc = row_wave(p.nTE, p.nTE, p.K, x.lamb1, x.fast, wave))) return rc;
+    const SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm, wave};
     const void *kern = g.kernel();
     if (!kern) return FG_OK;
     long long cap = 0;
-    const int rc = coresident_groups(kern, g.threads(), dev, cap);
+    rc = coresident_groups(kern, g.threads(), dev, cap);
     if (rc) return rc;
     if (max_groups > 0) cap = std::min<long long>(cap, max_groups);
     tiled = (long long)p.nTB * p.nTE <= cap;

@@ -115,7 +115,7 @@ def test_small_images(device, C, H, W, lamb):
 
 
 @pytest.mark.parametrize("lamb", [1.0, 0.5, 1.5])
-@pytest.mark.parametrize("K", [0, 6, 12, 18, 24])
+@pytest.mark.parametrize("K", [0, 6, 12, 18, 24, 30])
 def test_many_tiles(device, lamb, K):
     """Launches of more tiles than the front-and-producers form is used for:
     1-4 channels, initialising and later sweeps, lengths around one and two
@@ -160,3 +160,36 @@ def test_recording_time_grows_with_the_batch(device):
     few, many = took(1024), took(4096)
     print(f"1024 images {few * 1e3:.1f} ms, 4096 images {many * 1e3:.1f} ms", flush=True)
     assert many < 7 * few
+
+
+@pytest.mark.parametrize("lamb", [1.0, 0.5])
+@pytest.mark.parametrize("halo,shape", [(30, (9, 4000)), (24, (9, 9600)), (18, (40, 15000)), (30, (33, 1, 4000)),
+                                        (24, (9, 1, 9600)), (30, (34, 1, 2500)), (30, (2, 1, 2100)), (6, (13, 1, 40000))])
+def test_long_rows_at_a_requested_depth(device, halo, shape, lamb):
+    """Rows of more tiles than workgroups with a front and producers are
+    resident at the requested depth: 2D rows take a shallower depth, planes of
+    one row the one-wave form.  The stepper takes them (their first sweep is
+    tiled) and every result is the oracle's."""
+    rng = np.random.default_rng(halo + shape[-1])
+    img = rng.random((1, 1, *shape), dtype=np.float32)
+    m = (rng.random((1, 1, *shape)) > 0.001).astype(np.float32)
+    m[(0, 0) + tuple(rng.integers(0, s) for s in shape)] = np.nan
+    ti, tm = torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda()
+    sp = [1.5, 1.0, 0.7]
+    print(f"long rows halo={halo} {shape} lamb={lamb}", flush=True)
+    with np.errstate(all="ignore"):
+        want = (oracle.py_geodesic2d(img, m, 1e10, lamb, 1) if len(shape) == 2
+                else oracle.py_geodesic3d(img, m, sp, 1e10, lamb, 1))
+    old = FG.get_tuning()
+    FG.set_tuning(halo=halo)
+    try:
+        got = (FG.generalised_geodesic2d(ti, tm, 1e10, lamb, 1) if len(shape) == 2
+               else FG.generalised_geodesic3d(ti, tm, sp, 1e10, lamb, 1))
+        assert equal(got.cpu().numpy(), want)
+        st = FG.FastGeodisCpp.Stepper(64 << 20, 4, torch.cuda.current_device())
+        _, out = st.add(ti, tm, sp, 0, 1e10, lamb, 1.0 - lamb, 1)
+        while st.active():
+            st.step()
+        assert equal(out.cpu().numpy(), want)
+    finally:
+        FG.set_tuning(**old)
