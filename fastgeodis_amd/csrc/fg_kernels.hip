@@ -1510,8 +1510,13 @@ __device__ __forceinline__ void row_wave_run(const SweepDesc &Dd, const RowTile 
   }
 }
 
-template <bool LAMB1, bool FAST>
-__global__ __launch_bounds__(64) void row_wave_kernel(
+// MC: the most channels of a transform of the launch.  A kernel holds the
+// registers of its widest ring, and tiles wait for their neighbours, so a plane
+// of more tiles than are resident cannot run on it.  One kernel for 1-4 channels
+// took 118 registers (16 waves a CU); by MC 57-63, 63-70, 76-79, 77-79: 32, 28,
+// 24 and 24 waves, up to 8192 tiles of one channel (a line of 426 000).
+template <int MC, bool LAMB1, bool FAST>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MC == 1 ? 8 : MC == 2 ? 7 : 6))) void row_wave_kernel(
     const SweepDesc *__restrict__ descs, int ndesc, SweepDesc one, int K, unsigned tag_base,
     unsigned long long *__restrict__ halo_base, int *__restrict__ status, int spin_limit,
     unsigned *__restrict__ xhist) {
@@ -1537,7 +1542,7 @@ __global__ __launch_bounds__(64) void row_wave_kernel(
   // bytes, 33 slices to either side and stores based at 2^31 up to 32 of them
   // stay between the array's range and 2^32.
   static_assert(kRowWaveMaxK + kRowHaloStep - 3 <= 33 && kRowWaveMaxK <= 32, "slices past the ends stay out of range");
-  if (K <= 0 || K % kRowHaloStep != 0 || K > kRowWaveMaxK || Dd.nB != 1 || Dd.dxo || Dd.C < 1 || Dd.C > 4) {
+  if (K <= 0 || K % kRowHaloStep != 0 || K > kRowWaveMaxK || Dd.nB != 1 || Dd.dxo || Dd.C < 1 || Dd.C > MC) {
     if (threadIdx.x == 0) __hip_atomic_store(status, FG_EINVAL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return;
   }
@@ -1550,12 +1555,13 @@ __global__ __launch_bounds__(64) void row_wave_kernel(
     if (Dd.init_mode) row_wave_run<CT, LAMB1, FAST, true>(Dd, T, K, tag_base, halo, status, spin_limit, xh);
     else row_wave_run<CT, LAMB1, FAST, false>(Dd, T, K, tag_base, halo, status, spin_limit, xh);
   };
-  switch (Dd.C) {
-    case 1: run(std::integral_constant<int, 1>{}); break;
-    case 2: run(std::integral_constant<int, 2>{}); break;
-    case 3: run(std::integral_constant<int, 3>{}); break;
-    default: run(std::integral_constant<int, 4>{}); break;
-  }
+  if (MC == 1 || Dd.C == 1) run(std::integral_constant<int, 1>{});
+  if constexpr (MC > 1)
+    if (Dd.C == 2) run(std::integral_constant<int, 2>{});
+  if constexpr (MC > 2)
+    if (Dd.C == 3) run(std::integral_constant<int, 3>{});
+  if constexpr (MC > 3)
+    if (Dd.C == 4) run(std::integral_constant<int, 4>{});
   if (xhist) {
     __syncthreads();
     if (threadIdx.x < kXHistBuckets && xhist_wg[threadIdx.x]) atomicAdd(xhist + threadIdx.x, xhist_wg[threadIdx.x]);
@@ -2298,11 +2304,21 @@ const void *pick_row_variant(bool lamb1, bool fast) {
               : reinterpret_cast<const void *>(&row_sweep_kernel<K, false, false>);
 }
 
-const void *pick_row_kernel(int K, bool lamb1, bool fast, bool wave) {
-  if (wave) {
-    if (lamb1) return reinterpret_cast<const void *>(&row_wave_kernel<true, true>);
-    return fast ? reinterpret_cast<const void *>(&row_wave_kernel<false, true>)
-                : reinterpret_cast<const void *>(&row_wave_kernel<false, false>);
+template <int MC>
+const void *pick_row_wave(bool lamb1, bool fast) {
+  if (lamb1) return reinterpret_cast<const void *>(&row_wave_kernel<MC, true, true>);
+  return fast ? reinterpret_cast<const void *>(&row_wave_kernel<MC, false, true>)
+              : reinterpret_cast<const void *>(&row_wave_kernel<MC, false, false>);
+}
+
+// wave: 0, or the most channels of a launch on the one-wave form
+const void *pick_row_kernel(int K, bool lamb1, bool fast, int wave) {
+  switch (wave) {
+    case 1: return pick_row_wave<1>(lamb1, fast);
+    case 2: return pick_row_wave<2>(lamb1, fast);
+    case 3: return pick_row_wave<3>(lamb1, fast);
+    case 4: return pick_row_wave<4>(lamb1, fast);
+    default: break;
   }
   switch (K) {
     case 6: return pick_row_variant<6>(lamb1, fast);
@@ -2662,7 +2678,7 @@ struct SweepGroup {
   bool l1, fa;
   int xs;
   bool in, cm;
-  bool wave;  // rows: the one-wave form
+  int wave;  // rows on the one-wave form: the most channels of a transform
   bool row() const { return NW == 1; }
   int threads() const { return row() ? (wave ? 64 : kRowThreads) : (NW + (cm ? kCommWaves : 0)) * 64; }
   const void *kernel() const {
@@ -3020,7 +3036,7 @@ struct Runner {
   int row_wave(long long tiles, long long widest, int K, bool lamb1, bool fast, bool &wave) const {
     wave = tiles > (long long)kRowWaveTiles * dev.cus;
     if (wave || widest <= dev.cus) return FG_OK;  // (at least one a compute unit is resident)
-    const void *kern = pick_row_kernel(K, lamb1, fast, false);
+    const void *kern = pick_row_kernel(K, lamb1, fast, 0);
     long long cap = 0;
     if (!kern) return fail(FG_EINVAL, "no row kernel for this depth");
     if (const int rc = coresident_groups(kern, kRowThreads, dev, cap)) return rc;
@@ -3028,12 +3044,13 @@ struct Runner {
     return FG_OK;
   }
 
-  // Which of a pass's transforms run on it: the rows that share a launch (same
-  // depth, lamb class and fold) are counted together, once for the pass (a
+  // Which of a pass's transforms run on it (the most channels of its launch, or
+  // 0): the rows that share a launch (same depth, lamb class and fold) are
+  // counted together, once for the pass (a
   // count per transform made the recording of a batch quadratic: 1024 images of
   // 150 x 170 12.3 ms a call instead of 6.9).
   int row_waves(const std::vector<Xform *> &active, int pass, const std::vector<int> &ks, std::vector<char> &wave) const {
-    struct Launch { long long tiles = 0, widest = 0; bool wave = false; };
+    struct Launch { long long tiles = 0, widest = 0; int channels = 0; bool wave = false; };
     Launch launch[kMaxK + 1][2][2];
     wave.assign(active.size(), 0);
     for (size_t i = 0; i < active.size(); ++i) {
@@ -3046,6 +3063,7 @@ struct Runner {
       const int n = plan_fixed(nB, nE, ks[i], x->C).nTE;
       l.tiles += n;
       l.widest = std::max<long long>(l.widest, n);
+      l.channels = std::max(l.channels, x->C);
     }
     for (int k = 1; k <= kMaxK; ++k)
       for (int lamb1 = 0; lamb1 < 2; ++lamb1)
@@ -3054,8 +3072,11 @@ struct Runner {
           if (l.tiles == 0) continue;
           if (const int rc = row_wave(l.tiles, l.widest, k, lamb1, fast, l.wave)) return rc;
         }
-    for (size_t i = 0; i < active.size(); ++i)
-      wave[i] = wave[i] && launch[ks[i]][active[i]->lamb1][active[i]->fast].wave;
+    for (size_t i = 0; i < active.size(); ++i) {
+      if (!wave[i]) continue;
+      const Launch &l = launch[ks[i]][active[i]->lamb1][active[i]->fast];
+      wave[i] = l.wave ? (char)l.channels : 0;
+    }
     return FG_OK;
   }
 
@@ -3103,7 +3124,7 @@ struct Runner {
         }
         const bool row = p.NW == 1;
         const SweepGroup key{p.NW, p.R, p.P, p.K, row ? 0 : x->C, x->lamb1, x->fast, row ? 0 : xs, row ? false : in,
-                             p.comm, wave[i] != 0};
+                             p.comm, wave[i]};
         auto g = std::find_if(groups.begin(), groups.end(), [&](const auto &q) { return q.first == key; });
         if (g == groups.end()) g = groups.insert(groups.end(), {key, {}});
         g->second.push_back({x, pass, p.K, xs});
@@ -3139,6 +3160,13 @@ struct Runner {
       pass_plane(*j.x, j.pass, nA, nB, nE);
       Plan p = plan_fixed(nB, nE, j.K, j.x->C);
       const long long nt = (long long)p.nTB * p.nTE;
+      if (nt > cap && g.wave > j.x->C) {  // its own channel count's kernel holds more tiles
+        std::vector<SweepJob> alone{j};
+        SweepGroup own = g;
+        own.wave = j.x->C;
+        if ((rc = record_group(alone, dir, own))) return rc;
+        continue;
+      }
       if (nt > cap) {  // one plane alone cannot be co-resident: per-slice engine
         if (j.x->init_mode && j.x->it == 0 && j.pass == first_pass(*j.x) && dir > 0)
           return fail(FG_EINVAL, "internal: an initialising sweep was planned on the per-slice engine");
@@ -3295,7 +3323,7 @@ struct Runner {
     bool wave = false;
     int rc = FG_OK;
     if (nB == 1 && (rc = row_wave(p.nTE, p.nTE, p.K, x.lamb1, x.fast, wave))) return rc;
-    const SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm, wave};
+    const SweepGroup g{p.NW, p.R, p.P, p.K, x.C, x.lamb1, x.fast, 0, true, p.comm, wave ? x.C : 0};
     const void *kern = g.kernel();
     if (!kern) return FG_OK;
     long long cap = 0;

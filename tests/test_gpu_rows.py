@@ -193,3 +193,25 @@ def test_long_rows_at_a_requested_depth(device, halo, shape, lamb):
         assert equal(out.cpu().numpy(), want)
     finally:
         FG.set_tuning(**old)
+
+
+def test_widest_rows(device):
+    """Lines of more tiles than the one-wave form's kernel for 1-4 channels holds:
+    one channel's kernel holds twice as many.  Alone, beside an image with more
+    channels in one call, and on the stepper, which takes tiled sweeps only."""
+    rng = np.random.default_rng(31)
+    img, m = make(rng, 1, 5, 400000)
+    rgb, rm = make(rng, 3, 40, 70)
+    ti, tm = torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda()
+    want = oracle.py_geodesic2d(img, m, 1e10, 0.5, 1)
+    assert equal(FG.generalised_geodesic2d(ti, tm, 1e10, 0.5, 1).cpu().numpy(), want)
+    insts = [FG.Instance(ti, tm, 1e10, 0.5, iter=1),
+             FG.Instance(torch.from_numpy(rgb).cuda(), torch.from_numpy(rm).cuda(), 1e10, 0.5, iter=1)]
+    got = FG.geodesic_batch(insts)
+    assert equal(got[0].cpu().numpy(), want)
+    assert equal(got[1].cpu().numpy(), oracle.py_geodesic2d(rgb, rm, 1e10, 0.5, 1))
+    st = FG.FastGeodisCpp.Stepper(64 << 20, 4, torch.cuda.current_device())
+    _, out = st.add(ti, tm, [1.0, 1.0, 1.0], 0, 1e10, 0.5, 0.5, 1)
+    while st.active():
+        st.step()
+    assert equal(out.cpu().numpy(), want)
