@@ -253,13 +253,15 @@ __device__ __forceinline__ float min3(float a, float b, float c) {
   return r;
 }
 
-// The nine candidates of one row element in the order they become available:
-// rows[k] is the front row (B offset + 1) of the k-th triple.
+// The nine candidates of one row element, taken in triples of a front row as
+// they become available.
 // FAST: folded with IEEE minNum as they come (any order gives the same value,
-// as no candidate is -0); otherwise kept for the reference's order.
+// as no candidate is -0); otherwise kept for the reference's order, and folded
+// in it as far as they are there (`early`).
 template <bool FAST>
 struct Fold {
   float c[9];   // !FAST: candidate of front row i, lane offset j at i * 3 + j
+  float nd;     // !FAST: the old value and the first candidates folded
   float m;      // FAST: minimum so far
   float left;   // FAST: a candidate that waits for the next pair
   int n = 0;    // triples taken
@@ -278,12 +280,21 @@ struct Fold {
       for (int j = 0; j < 3; ++j) c[i * 3 + j] = t[j];
     }
   }
-  __device__ __forceinline__ float with(float dinit) const {
-    if constexpr (FAST) return (m < dinit) ? m : dinit;
-    float nd = dinit;
+  // !FAST: folds the first k candidates (all taken by then)
+  __device__ __forceinline__ void early(float dinit, int k) {
+    nd = dinit;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) nd = (c[k] < nd) ? c[k] : nd;
-    return nd;
+    for (int q = 0; q < 9; ++q)
+      if (q < k) nd = (c[q] < nd) ? c[q] : nd;
+  }
+  // the new value; k: candidates that `early` folded (0: it was not called)
+  __device__ __forceinline__ float with(float dinit, int k) const {
+    if constexpr (FAST) return (m < dinit) ? m : dinit;
+    float v = k ? nd : dinit;
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+      if (q >= k) v = (c[q] < v) ? c[q] : v;
+    return v;
   }
 };
 
@@ -940,6 +951,14 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
     constexpr std::integral_constant<int, 0> above{};
     constexpr std::integral_constant<int, 1> same{};
     constexpr std::integral_constant<int, 2> below{};
+    // Candidates of row r, first in the reference's order, that are folded
+    // before the barrier: the row then holds one value over it instead.  Where
+    // registers decide how many workgroups a unit holds: 8 x 4 with 4 channels
+    // takes 124 of them instead of 132 (two workgroups, else one), 4 x 8 with 2
+    // channels 140 instead of 184 (three, else two).  Elsewhere it is no gain
+    // (lamb 1.5, 20 x 120 x 140 888 / 910 us, 256 x 400 x 400 4187 / 4231).
+    constexpr bool kEarly = !FAST && P == 2 && (R == 8 || CT == 4);
+    auto early_of = [](int r) { return !kEarly || r == 0 ? 0 : r < R - 1 ? 9 : 6; };
     const bool live = j <= live_steps;
     if (live) {
 #pragma unroll
@@ -947,6 +966,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
         triple(same, r, Fd[r]);
         if (r > 0) triple(above, r, Fd[r - 1]);
         if (r < R - 1) triple(below, r, Fd[r + 1]);
+        if (early_of(r) > 0) fold[r].early(init_of(Sl.d[r]), early_of(r));
       }
     }
     __builtin_amdgcn_sched_barrier(0);  // (the compiler would move these past the barrier)
@@ -965,7 +985,7 @@ __global__ __launch_bounds__((NW + (COMM ? kCommWaves : 0)) * 64) void sweep_til
       triple(below, R - 1, (w < w_last) ? u : kInf);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const float v = fold[r].with(init_of(Sl.d[r]));
+        const float v = fold[r].with(init_of(Sl.d[r]), early_of(r));
         Fd[r] = pvalid[r] ? v : kInf;
       }
     }

@@ -42,3 +42,29 @@ def test_rows(device, halo, shape, lamb, C):
             assert equal(got.cpu().numpy(), want)
     finally:
         FG.set_tuning(**old)
+
+
+@pytest.mark.parametrize("shape,C,dims", [(2, 4, (2, 700, 800)), (1, 2, (2, 900, 1200))])
+def test_wide_planes_in_the_reference_order(device, shape, C, dims):
+    """Planes of 350 and 660 tiles with lamb > 1 (candidates kept for the
+    reference's order): two and three workgroups a compute unit are resident, so
+    the sweeps are tiled and the stepper takes them."""
+    rng = np.random.default_rng(shape)
+    img = rng.random((1, C, *dims), dtype=np.float32)
+    m = (rng.random((1, 1, *dims)) > 0.01).astype(np.float32)
+    m[0, 0, 0, 100, 100] = np.nan
+    sp = [1.5, 1.0, 0.7]
+    ti, tm = torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda()
+    with np.errstate(all="ignore"):
+        want = oracle.py_geodesic3d(img, m, sp, 1e10, 1.25, 1)
+    old = FG.get_tuning()
+    FG.set_tuning(shape=shape)
+    try:
+        assert equal(FG.generalised_geodesic3d(ti, tm, sp, 1e10, 1.25, 1).cpu().numpy(), want)
+        st = FG.FastGeodisCpp.Stepper(64 << 20, 4, torch.cuda.current_device())
+        _, out = st.add(ti, tm, sp, 0, 1e10, 1.25, 1.0 - 1.25, 1)
+        while st.active():
+            st.step()
+        assert equal(out.cpu().numpy(), want)
+    finally:
+        FG.set_tuning(**old)
