@@ -215,3 +215,32 @@ def test_widest_rows(device):
     while st.active():
         st.step()
     assert equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("lamb", [1.0, 0.5, 1.5])
+@pytest.mark.parametrize("what", ["signed", "gsf", "gsf-second-stage", "mixed"])
+def test_many_tiles_of_signed_and_filtered_images(device, what, lamb):
+    """Signed transforms and the filter on the one-wave form: both ways to
+    initialise, the epilogues' combining transposes after sweeps that write their
+    own layout, images of both orientations.  gsf-second-stage: 12 images of 30
+    tiles (K = 12) are 720 tiles in the first stage, on the front-and-producers
+    form, and 1152 (of 24, K = 6) in the second."""
+    rng = np.random.default_rng(len(what))
+    insts, wants = [], []
+    for k in range(12 if what == "gsf-second-stage" else 44):
+        C, n = 1 + k % 4, (2, 7, 13, 26)[k % 4]
+        op = {"mixed": ("unsigned", "signed", "gsf")[k % 3]}.get(what, what.split("-")[0])
+        H, W = (n, 1190) if what == "gsf-second-stage" or k % 2 else (1190 + k, n)
+        img, _ = make(rng, C, H, W)
+        m = (rng.random((1, 1, H, W)) > 0.4).astype(np.float32)
+        it = 2 + k % 2
+        wants.append({"unsigned": lambda: oracle.py_geodesic2d(img, m, 1e10, lamb, it),
+                      "signed": lambda: oracle.py_signed_geodesic2d(img, m, 1e10, lamb, it),
+                      "gsf": lambda: oracle.py_gsf2d(img, m, 0.1, 1e10, lamb, it)}[op]())
+        insts.append(FG.Instance(torch.from_numpy(img).cuda(), torch.from_numpy(m).cuda(), 1e10, lamb, iter=it, op=op,
+                                 theta=0.1))
+    if what != "gsf-second-stage":
+        insts, wants = insts + insts, wants + wants  # (> 2000 tiles of rows and of columns)
+    print(f"many tiles {what} lamb={lamb}", flush=True)
+    for got, want in zip(FG.geodesic_batch(insts), wants):
+        assert equal(got.cpu().numpy(), want)
