@@ -3054,6 +3054,7 @@ struct Runner {
   // than workgroups with a front and producers are resident at once (512 at
   // K >= 24; a requested depth can ask for it).
   int row_wave(long long tiles, long long widest, int K, bool lamb1, bool fast, bool &wave) const {
+    if (max_groups > 0) tiles = std::min<long long>(tiles, max_groups);  // a launch has no more
     wave = tiles > (long long)kRowWaveTiles * dev.cus;
     if (wave || widest <= dev.cus) return FG_OK;  // (at least one a compute unit is resident)
     const void *kern = pick_row_kernel(K, lamb1, fast, 0);
