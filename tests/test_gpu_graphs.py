@@ -32,6 +32,9 @@ CALLS = [
     ("signed3d", lambda i, m, lamb: FG.signed_generalised_geodesic3d(i, m, [1.0, 1.0, 1.0], 1e10, lamb, 2),
      (20, 64, 80)),
     ("gsf2d", lambda i, m, lamb: FG.GSF2d(i, m, 0.1, 1e10, lamb, 2), (128, 160)),
+    # whole transforms in one workgroup, with most of a compute unit's LDS
+    ("small2d", lambda i, m, lamb: FG.generalised_geodesic2d(i, m, 1e10, lamb, 2), (127, 128)),
+    ("smallgsf2d", lambda i, m, lamb: FG.GSF2d(i, m, 0.1, 1e10, lamb, 2), (64, 90)),
 ]
 
 
