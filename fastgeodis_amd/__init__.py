@@ -226,11 +226,12 @@ def transposed_image(image: torch.Tensor) -> torch.Tensor:
 def set_tuning(engine: int = 1, halo: int = 0, max_groups: int = 0, shape: int = 0) -> None:
     """Engine (0 per-slice, 1 persistent tiled), halo depth K (slices between
     neighbour exchanges; 0 = automatic: the deepest halo whose tiles fit the
-    device), workgroup cap (0 = occupancy limit) and 3D plane workgroup shape
-    (0 auto: 5, or 7 for passes whose planes fit the device with it; 1 = 4
-    waves x 8 rows, 2 = 8 x 4, 3 = 16 x 2, 4 = 8 x 4 with a deeper prefetch ring, 5 = 16 x 2 with the deeper ring,
-    6 = 8 x 4 with the deeper ring and four more waves that perform the halo
-    exchanges, 7 = 8 waves x 2 rows, a 16-row window, with the deeper ring)
+    device and the workgroup cap), workgroup cap of a launch (0 = occupancy
+    limit) and 3D plane workgroup shape (0 auto: 5, or 7 for passes whose planes
+    fit the device with it; 1 = 4 waves x 8 rows, 2 = 8 x 4, 3 = 16 x 2, 4 = 8 x 4
+    with a deeper prefetch ring, 5 = 16 x 2 with the deeper ring, 6 = 8 x 4 with
+    the deeper ring and four more waves that perform the halo exchanges, 7 = 8
+    waves x 2 rows, a 16-row window, with the deeper ring)
     used by later calls on this host thread."""
     FastGeodisCpp.set_tuning(int(engine), int(halo), int(max_groups), int(shape))
 

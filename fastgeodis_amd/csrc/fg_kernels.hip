@@ -16,11 +16,13 @@
 //           per call; the distance enters that layout through the H pass's
 //           backward sweep, which writes it directly, and leaves it through
 //           the W pass's backward sweep, which writes the native layout; a
-//           transpose instead where those forms do not apply (3-4 channels,
-//           other shapes and halo depths) and after a signed or GSF
-//           transform's last W pass, where it applies the epilogue)
+//           transpose instead where those forms do not apply (3-4 channels, 2
+//           channels on the automatic shapes, other shapes, the W pass at
+//           K > 5) and after a signed or GSF transform's last W pass, where it
+//           applies the epilogue)
 //   2D: rows A=H, E=W on (H,W); columns A=W, E=H on (W,H), the backward row
-//       and column sweeps writing the other layout
+//       and column sweeps writing the other layout (through transposes in
+//       launches of many row tiles, kRowWaveTiles)
 // B and E are the reference's in-plane axes in its neighbour order (B outer,
 // E inner), so the exact-order path visits candidates in the reference order.
 //
@@ -314,6 +316,10 @@ typedef __attribute__((address_space(1))) unsigned long long gu64;
 // flight together (under branches the compiler waited for each row's load
 // before it issued the next one).  The offsets fit 32 bits: the tiles of a
 // launch are resident together, and each has two slots of less than 64 KB.
+// They are plain stores and loads, not atomics: what the exchange rests on is
+// that the aligned 8 bytes that one lane's instruction writes become visible
+// whole, so a reader that sees the tag has the value.  Nothing else is ordered
+// by an entry, so there is no release or acquire.
 constexpr unsigned kNoHalo = 0xFFFFFFFFu;
 constexpr int kHaloCache = 16;  // sc1
 typedef unsigned uint2v __attribute__((ext_vector_type(2)));
@@ -1637,7 +1643,14 @@ struct SmallElement<4> { typedef float4 type; };
 // to 64 elements is one wave's, a longer one is split over up to four waves
 // with 32 own lanes each and 16 lanes of halo to either side, which are read
 // back from the lines in LDS every 16 steps behind a barrier.  64^2, one
-// channel, iter 2: 73 -> 33 us a call; 128^2 98 -> 78 us.
+// channel, iter 2: 73 -> 33 us a call; 128^2 98 -> 78 us.  A step takes 53-58 ns
+// (3 channels 90), as its image term is on the chain; up to a side of 64 one
+// wave of the four walks it.
+// Between barriers a wave's halo lanes may read a line's old distances after
+// the wave that owns them has replaced them.  That changes no result: a halo
+// lane that still counts computes the same minimum from the replaced value (it
+// is the minimum of the old one and the same candidates, and is kept by both
+// folds), and the others reach no own lane before they are read back.
 template <int CT, bool LAMB1, bool FAST>
 __global__ __launch_bounds__(kSmallWaves * 64) void small_call_kernel(const SmallDesc *__restrict__ descs,
                                                                       SmallDescs few) {
@@ -2685,10 +2698,12 @@ struct SweepJob {
 
 // Row launches of more tiles than this a compute unit run the one-wave form.
 // Front and producers / one wave, ms a call: 32 RGB 1024^2 GSF iter 4 (2560
-// tiles) 31.4 / 20.3, 64 of 512^2 (832) 1.31 / 1.20; below the line a
-// 1252 x 1292 GSF (324 tiles at K = 24) 1.3 / 2.1.  The one-wave form's tiles
-// leave the layout change to transposes: storing the other layout themselves
-// (runs of K elements a lane) they took 28.8 ms on the first.
+// tiles) 31.4 / 20.0, 64 of 512^2 (832) 1.31 / 1.18; below the line a
+// 1252 x 1292 GSF (324 tiles at K = 24) 1.3 / 2.1.  (One-wave tiles were the
+// only form once and took 20.0 and 1.22 there: above the line nothing is
+// gained, below it the front wave's shorter chain is.)  The one-wave form's
+// tiles leave the layout change to transposes: storing the other layout
+// themselves (runs of K elements a lane) they took 28.8 ms on the first.
 constexpr int kRowWaveTiles = 3;
 
 // What the sweeps of one launch share.  Row sweeps (row()) of any channel
@@ -2765,9 +2780,11 @@ struct Runner {
   }
 
   // Whether the H-backward sweep of this transform can write the transposed
-  // layout itself: 3D, tiled engine with the default shape and a
-  // transposed-output kernel for its channel count, and every output offset
-  // within 32 bits.
+  // layout itself: 3D, tiled engine, a B-contiguous kernel for its channel count
+  // on the thread's shape, and every output offset within 32 bits.  The pass may
+  // still run on 16-row windows, and the choice is made again when it is
+  // recorded; with the automatic shape two channels never get here (16 x 2 has
+  // no such kernel for them), and their distance is transposed.
   bool xstore_candidate(const Xform &x) {
     if (x.is2d) return row_xsa_candidate(x, 1);
     if (engine == 0 || x.C > kXstMaxC) return false;
@@ -2798,10 +2815,10 @@ struct Runner {
   }
 
   // 2D: whether the backward sweep of rows (pass 1) may write the column
-  // layout, or that of columns (pass 2) the native layout, itself; the
-  // launch then also needs the one-row kernel whose block is one turn of its
-  // 30-slice ring (checked when it is recorded).  The output, like the input,
-  // is addressed with 32-bit offsets within 2^31 bytes.
+  // layout, or that of columns (pass 2) the native layout, itself; the launch
+  // must also run the front-and-producers form (decided when it is recorded).
+  // The output, like the input, is addressed with 32-bit offsets within 2^31
+  // bytes.
   bool row_xsa_candidate(const Xform &x, int pass) {
     if (engine == 0 || x.C > 4) return false;
     int nA, nB, nE;
@@ -3158,7 +3175,10 @@ struct Runner {
     return FG_OK;
   }
 
-  // A group is split into launches whose tiles can all be co-resident.
+  // A group is split into launches whose tiles can all be co-resident.  For the
+  // automatic 3D shape that is one workgroup a compute unit, as its kernels take
+  // more than 64 registers (65-97); two in turn finish sooner than two at once
+  // (clicks in eight volumes 10.27 / 11.21 ms).
   int record_group(std::vector<SweepJob> &jobs, int dir, const SweepGroup &g) {
     const void *kern = g.kernel();
     if (!kern) return fail(FG_EINVAL, "no tiled kernel for this shape");
@@ -3601,9 +3621,14 @@ bool small_op(const OpSpec &o) {
   return o.is2d && o.iters > 0 && side <= (o.C == 1 ? kSmallSide : 64) && o.C <= 3 && g_tune.engine != 0 &&
          g_tune.halo == 0 && g_tune.max_groups == 0 && small_lds(o.C, o.H, o.W) <= (160u << 10);
 }
-// They do when all ops of the call can: beside larger ones they share those
-// launches at no cost of their own (a batch of 48 images and 8 volumes: 4735
-// us, 4896 with its small images in launches of their own).
+// They do when all ops of the call can, however many there are: workgroups of
+// more than 80 KB (a side of ~96) take a compute unit each, so large batches run
+// in rounds of 256, and still take less than their sweeps would, host time
+// included.  Calls of n images, this kernel / sweeps, us: 128^2, n = 64 327 /
+// 443, 256 990 / 1403, 1024 3916 / 5091; GSF 256 1663 / 3765; 90^2, 1024 3916 /
+// 5007; 3 channels of 64^2, 1024 3791 / 5110.  Beside larger images they share
+// those launches at no cost of their own (a batch of 48 images and 8 volumes:
+// 4735 us, 4896 with its small images in launches of their own).
 bool small_ops(const std::vector<OpSpec> &ops) { return std::all_of(ops.begin(), ops.end(), small_op); }
 
 int n_dist(int op) { return op == FG_OP_UNSIGNED ? 1 : (op == FG_OP_SIGNED ? 2 : 4); }

@@ -220,17 +220,19 @@ int fg_set_voxels_f32(const fg_voxel_set *items, int n, void *stream);
 /* Tile/launch parameters of the persistent sweep engine.  engine 0 is the
  * one-launch-per-slice engine, 1 the persistent tiled engine (default).
  * halo is the trapezoid depth K (slices per neighbour exchange, 1..30),
- * rounded up to a multiple of the kernel's slab ring; 0 (default) picks the
- * deepest halo whose tiles fit the device (3D tiles one per compute unit, 2D
- * row tiles one to four): per 2D row and per lone 3D plane, and over all 3D
- * planes that share a pass (batches, the halves of a signed or GSF call).  Values are per host thread; fg_tuning_get reads
- * them back. */
+ * rounded up to a multiple of the kernel's slab ring (2D rows that are too many
+ * for it take a shallower one); 0 (default) picks the deepest halo whose tiles
+ * fit the device (3D tiles one per compute unit, 2D row tiles one to four) and
+ * max_groups: for a lone 2D row or 3D plane alone, and over all rows or planes
+ * that share a pass (batches, the halves of a signed or GSF call).  Values are
+ * per host thread; fg_tuning_get reads them back. */
 typedef struct fg_tuning {
   int engine;
   int halo;
   int max_groups; /* cap on persistent workgroups (0 = occupancy limit) */
   int shape;      /* 3D plane workgroup shape (waves x rows / slab ring): 0 auto
-                     (5, or 7 for passes whose planes fit the device with it), 1 = 4x8/2, 2 = 8x4/3, 3 = 16x2/3, 4 = 8x4/5, 5 = 16x2/5,
+                     (5, or 7 for passes whose planes fit the device with it),
+                     1 = 4x8/2, 2 = 8x4/3, 3 = 16x2/3, 4 = 8x4/5, 5 = 16x2/5,
                      6 = 8x4/5 plus four waves that perform the halo exchanges
                      (1-2 channels; 3-4 channels run 8x4/2), 7 = 8x2/5 (16-row
                      windows; 3-4 channels 8x2/3) */
